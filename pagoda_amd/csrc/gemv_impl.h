@@ -444,8 +444,8 @@ bool q6k_mma_ok(const GemvArgs& a, int epi);
 void run_q6k_mma(const GemvArgs& a, int nrows, int x_f16, int epi, hipStream_t s);
 // Per-stream device scratch that grows on demand (the stream is synchronized
 // before a buffer is replaced). Slots are independent buffers: 0 for prepared
-// activations and small reductions, 1 for split-K partial sums, 3 for
-// stream-K partial sums, 4 for attention chunk states, 5 for per-row scales.
+// activations and small reductions, 1 for split-K partial sums, 2 for Q8_K
+// activation operands, 3 for stream-K partial sums, 4 for attention chunk states, 5 for per-row scales.
 void* gemv_scratch(hipStream_t s, size_t bytes, int slot = 0);
 // device scratch bytes (with per-slot alignment) one prepared-activation A8
 // GEMV of `rows` rows takes through run_a8_mma (epi EPI_STORE or EPI_RES, no
@@ -456,6 +456,9 @@ void sk_scratch_need(const GemvArgs& a, int nb, int epi, size_t* slot3, size_t* 
 // GGML formats with candle's CPU arithmetic (activations quantized to Q8_K /
 // Q8_0, integer block dots); f32 activations
 void run_q8act(int fmt, const GemvArgs& a, int nrows, int epi, hipStream_t s);
+// the same outputs for many rows of Q4_K / Q6_K matrices on the matrix cores
+void run_q8_gemm(int fmt, GemvArgs a, int nrows, int epi, hipStream_t s);
+void run_q8_gemm_pair(int fmt_a, GemvArgs a, int fmt_b, GemvArgs b, int nrows, hipStream_t s);
 // two store GEMVs of one input in one launch (formats of one activation type)
 bool q8act_pair_ok(int fmt_a, int fmt_b);
 void run_q8act_pair(int fmt_a, const GemvArgs& a, int fmt_b, const GemvArgs& b, int nrows, hipStream_t s);

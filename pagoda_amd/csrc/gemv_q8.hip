@@ -29,6 +29,9 @@
 // them in block order. The per-row arithmetic does not depend on the number
 // of rows, so batched rows are bitwise equal to single-row launches.
 //
+// Launches of kGemmRows or more rows of Q4_K / Q6_K matrices run on the matrix
+// cores instead (gemm_q8.hip, the same bits).
+//
 // Work split: one workgroup of NW waves (4 or 8, from the number of K
 // blocks) per 32-row tile of the weight matrix; wave w takes K blocks w,
 // w + NW, ... (256-element super-blocks, or 32-weight blocks). Weights are
@@ -584,6 +587,13 @@ size_t lds_need(int n_in, int nm) {
   return ActLds<FMT, RB, 8>::bytes(n_in, nm);
 }
 
+// Rows from which Q4_K / Q6_K launches run on the matrix cores (gemm_q8.hip),
+// whose second launch (the activation operands) costs about 2 us: at 3 rows
+// the two paths measured within 6% of each other either way over the 0.5B
+// model's shapes, at 4 rows the matrix cores were 1.10..1.40x faster on all
+// of them, at 16 rows 2.8..5x.
+constexpr int kGemmRows = 4;
+
 // rows per launch: decode steps take 1..8; prefills 16 at a time (weights
 // read once per 16 rows). Wide rows whose RB quantized rows do not fit the
 // 160 KiB of LDS take fewer rows per launch (the per-row arithmetic does not
@@ -592,8 +602,15 @@ template <int FMT, int EPI>
 void launch_rows(const GemvArgs& a, int nrows, hipStream_t s) {
   const int nm = EPI == EPI_SWIGLU ? 2 : 1;
   const size_t cap = 160 * 1024;
-  if (nrows > 8 && lds_need<FMT, 16>(a.n_in, nm) <= cap) return launch_waves<FMT, 16, EPI>(a, nrows, s);
-  if (nrows > 4 && lds_need<FMT, 8>(a.n_in, nm) <= cap) return launch_waves<FMT, 8, EPI>(a, nrows, s);
+  if constexpr (FMT == FMT_Q4K || FMT == FMT_Q6K) {
+    // one width limit for every row count
+    PGD_CHECK((lds_need<FMT, 1>(a.n_in, nm)) <= cap, kErrShape,
+              "activation rows too wide for the quantized-activation GEMV");
+    if (nrows >= kGemmRows) return run_q8_gemm(FMT, a, nrows, EPI, s);
+  } else {
+    if (nrows > 8 && lds_need<FMT, 16>(a.n_in, nm) <= cap) return launch_waves<FMT, 16, EPI>(a, nrows, s);
+    if (nrows > 4 && lds_need<FMT, 8>(a.n_in, nm) <= cap) return launch_waves<FMT, 8, EPI>(a, nrows, s);
+  }
   if (nrows > 1 && lds_need<FMT, 4>(a.n_in, nm) <= cap) return launch_waves<FMT, 4, EPI>(a, nrows, s);
   launch_waves<FMT, 1, EPI>(a, nrows, s);
 }
@@ -648,8 +665,14 @@ void pair_rows(const GemvArgs& a, const GemvArgs& b, int nrows, hipStream_t s) {
     constexpr int RB = decltype(rb)::value;
     return lds_need<FMT, RB>(a.n_in, 1) <= cap && lds_need<FMT2, RB>(a.n_in, 1) <= cap;
   };
-  if (nrows > 8 && fits(std::integral_constant<int, 16>{})) return go(std::integral_constant<int, 16>{});
-  if (nrows > 4 && fits(std::integral_constant<int, 8>{})) return go(std::integral_constant<int, 8>{});
+  if constexpr (FMT == FMT_Q4K || FMT == FMT_Q6K) {
+    PGD_CHECK(fits(std::integral_constant<int, 1>{}), kErrShape,
+              "activation rows too wide for the quantized-activation GEMV");
+    if (nrows >= kGemmRows) return run_q8_gemm_pair(FMT, a, FMT2, b, nrows, s);
+  } else {
+    if (nrows > 8 && fits(std::integral_constant<int, 16>{})) return go(std::integral_constant<int, 16>{});
+    if (nrows > 4 && fits(std::integral_constant<int, 8>{})) return go(std::integral_constant<int, 8>{});
+  }
   if (nrows > 1 && fits(std::integral_constant<int, 4>{})) return go(std::integral_constant<int, 4>{});
   go(std::integral_constant<int, 1>{});
 }

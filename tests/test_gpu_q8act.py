@@ -156,3 +156,58 @@ def test_q8act_wide_rows_16(dev, fmt, n_in):
     for p in (xd, yd, y1):
         dev.free(p)
     m.free()
+
+
+def extreme_blocks(rng, fmt, n_out, n_in):
+    """Blocks of random bytes (every scale, min and code) at a moderate d, the
+    first rows all at the ends of the integer ranges."""
+    nsb = (n_in + 255) // 256
+    d = np.frombuffer(np.float16(2e-4).tobytes(), np.uint8)
+    if fmt == 1:
+        b = rng.integers(0, 256, (n_out, nsb, 144)).astype(np.uint8)
+        b[0, :, 4:] = 0xFF  # scales and mins 63, codes 15
+        b[:, :, 0:2] = b[:, :, 2:4] = d
+    else:
+        b = rng.integers(0, 256, (n_out, nsb, 210)).astype(np.uint8)
+        b[:2, :, :192] = 0  # codes -32
+        b[0, :, 192:208] = 0x80  # scales -128
+        b[1, :, 192:208] = 0x8F  # -113: -128 and +15 in the two operands
+        b[:, :, 208:] = d
+    return b
+
+
+@pytest.mark.parametrize("fmt", [1, 2])
+@pytest.mark.parametrize("n_out,n_in,rows", [
+    (40, 320, 4),       # the fewest rows; a K tail; partly filled weight subtile and tile
+    (16, 256, 16),      # one subtile, one block, one whole activation tile
+    (129, 1280, 17),    # one row into the second activation tile
+    (3216, 896, 161),   # two activation tiles per workgroup, the last group's second one missing
+    (48, 512, 1027),    # rows past one prepared chunk
+])
+def test_q8act_many_rows_matches_oracle(dev, fmt, n_out, n_in, rows):
+    """The matrix-core path: bit-equal to the oracle at the edges of its tiles
+    and at the largest integers (class sums of 2^24), and to its own pair form."""
+    from pagoda_amd import Matrix
+
+    rng = np.random.default_rng(n_out + rows)
+    blk = extreme_blocks(rng, fmt, n_out, n_in)
+    m = Matrix.upload_kq(dev, fmt, blk, n_out, n_in)
+    x = rng.normal(0, 1, (rows, n_in)).astype(np.float32)
+    x[0] = 3.0   # every q is -128
+    x[1] = 0.0
+    x[2, ::8] = -100.0  # one residue class carries each block
+    xd, yd, y2 = dev.upload(x), dev.alloc(rows * n_out * 4), dev.alloc(rows * 2 * n_out * 4)
+    ref = oracle_rows(fmt, blk, n_out, n_in, x)
+    m.gemv_q8act_dev(xd, n_in, rows, yd, n_out)
+    got = dev.download(yd, (rows, n_out), np.float32)
+    assert close(got, ref), (np.abs(got - ref).max(), int((got != ref).sum()))
+    res = rng.normal(0, 1, (rows, n_out)).astype(np.float32)
+    rd = dev.upload(res)
+    m.gemv_q8act_dev(xd, n_in, rows, rd, n_out, rd, n_out)
+    assert close(dev.download(rd, (rows, n_out), np.float32), res + ref)
+    m.gemv_q8act_pair_dev(y2, m, y2 + n_out * 4, xd, n_in, rows, 2 * n_out)
+    pair = dev.download(y2, (rows, 2 * n_out), np.float32)
+    assert close(pair[:, :n_out], ref) and close(pair[:, n_out:], ref)
+    for p in (xd, yd, y2, rd):
+        dev.free(p)
+    m.free()
