@@ -456,7 +456,9 @@ void sk_scratch_need(const GemvArgs& a, int nb, int epi, size_t* slot3, size_t* 
 // GGML formats with candle's CPU arithmetic (activations quantized to Q8_K /
 // Q8_0, integer block dots); f32 activations
 void run_q8act(int fmt, const GemvArgs& a, int nrows, int epi, hipStream_t s);
-// the same outputs for many rows of Q4_K / Q6_K matrices on the matrix cores
+// Q4_K / Q6_K: a few rows, and any number of rows on the matrix cores
+void run_q8k_gemv(int fmt, const GemvArgs& a, int nrows, int epi, hipStream_t s);
+void run_q8k_gemv_pair(int fmt_a, const GemvArgs& a, int fmt_b, const GemvArgs& b, int nrows, hipStream_t s);
 void run_q8_gemm(int fmt, GemvArgs a, int nrows, int epi, hipStream_t s);
 void run_q8_gemm_pair(int fmt_a, GemvArgs a, int fmt_b, GemvArgs b, int nrows, hipStream_t s);
 // two store GEMVs of one input in one launch (formats of one activation type)

@@ -178,15 +178,20 @@ def extreme_blocks(rng, fmt, n_out, n_in):
 
 @pytest.mark.parametrize("fmt", [1, 2])
 @pytest.mark.parametrize("n_out,n_in,rows", [
-    (40, 320, 4),       # the fewest rows; a K tail; partly filled weight subtile and tile
+    (40, 320, 1),       # one row; a K tail; partly filled weight tile
+    (40, 320, 4),       # the most rows of the vector-ALU kernel
+    (40, 320, 5),       # the fewest on the matrix cores
+    (33, 4864, 6),      # 19 blocks over 10 waves, 6 rows
+    (33, 18944, 2),     # 74 blocks: rows one launch at a time
+    (33040, 256, 1),    # more tiles than workgroups
     (16, 256, 16),      # one subtile, one block, one whole activation tile
     (129, 1280, 17),    # one row into the second activation tile
     (3216, 896, 161),   # two activation tiles per workgroup, the last group's second one missing
     (48, 512, 1027),    # rows past one prepared chunk
 ])
-def test_q8act_many_rows_matches_oracle(dev, fmt, n_out, n_in, rows):
-    """The matrix-core path: bit-equal to the oracle at the edges of its tiles
-    and at the largest integers (class sums of 2^24), and to its own pair form."""
+def test_q8act_kernels_match_oracle(dev, fmt, n_out, n_in, rows):
+    """Both K-quant kernels: bit-equal to the oracle at the edges of their tiles
+    and at the largest integers (class sums of 2^24), and to their pair form."""
     from pagoda_amd import Matrix
 
     rng = np.random.default_rng(n_out + rows)
@@ -194,8 +199,8 @@ def test_q8act_many_rows_matches_oracle(dev, fmt, n_out, n_in, rows):
     m = Matrix.upload_kq(dev, fmt, blk, n_out, n_in)
     x = rng.normal(0, 1, (rows, n_in)).astype(np.float32)
     x[0] = 3.0   # every q is -128
-    x[1] = 0.0
-    x[2, ::8] = -100.0  # one residue class carries each block
+    x[1:2] = 0.0
+    x[2:3, ::8] = -100.0  # one residue class carries each block
     xd, yd, y2 = dev.upload(x), dev.alloc(rows * n_out * 4), dev.alloc(rows * 2 * n_out * 4)
     ref = oracle_rows(fmt, blk, n_out, n_in, x)
     m.gemv_q8act_dev(xd, n_in, rows, yd, n_out)
