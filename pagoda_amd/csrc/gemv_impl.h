@@ -71,6 +71,10 @@ struct GemvArgs {
   size_t coff;
   float* cout;
   int ldc, conv_n, conv_k;
+  // quantized-activation launches of a few rows (null: none): the input is
+  // x / rms(x) * norm_w, candle's rms_norm with its order of additions
+  const float* norm_w;
+  float norm_eps;
 };
 
 // the causal conv step of one channel for one row: conv_step_kernel's
@@ -464,6 +468,12 @@ void run_q8_gemm_pair(int fmt_a, GemvArgs a, int fmt_b, GemvArgs b, int nrows, h
 // two store GEMVs of one input in one launch (formats of one activation type)
 bool q8act_pair_ok(int fmt_a, int fmt_b);
 void run_q8act_pair(int fmt_a, const GemvArgs& a, int fmt_b, const GemvArgs& b, int nrows, hipStream_t s);
+// whether launches of nrows rows over tiles16 16-row tiles (nm matrices) can
+// run the input's RMSNorm themselves (GemvArgs.norm_w), and whether that pays:
+// every workgroup repeats the chain of n_in additions, so only while all of
+// them are resident at once
+bool q8k_norm_ok(int tiles16, int nsb, int n_in, int nrows, int nm);
+bool q8act_norm_fused(int fmt, int tiles16, int nsb, int n_in, int nrows, int nm);
 // A8 on the matrix cores (f32 activations)
 void run_a8_mma(const GemvArgs& a, const A8Act& act, int epi, hipStream_t s);
 // A8 GEMM for prefill-sized batches: rows [0, rows) of a prepared activation

@@ -54,9 +54,43 @@ struct Planes {
   const uint8_t *p0, *p1, *p2, *p3;
 };
 
+// floats of one row's squares: whole rounds of 64 and one more that the last
+// round's prefetch reads
+__host__ __device__ inline int sq_stride(int n) { return ((n + 63) & ~63) + 64; }
+
+// ((0 + q[0]) + q[1]) + ... over np (a multiple of 64) floats in LDS: the reads
+// of 32 in flight under the additions of the 32 before (rmsnorm_ordered_kernel)
+__device__ inline float ordered_sum(const float* q0, int np) {
+  const f4* q = reinterpret_cast<const f4*>(q0);
+  float ss = 0.0f;
+  auto read = [&](f4 (&v)[8], int i) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = q[i + k];
+  };
+  auto add = [&](const f4 (&v)[8]) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      ss += v[k][0];
+      ss += v[k][1];
+      ss += v[k][2];
+      ss += v[k][3];
+    }
+  };
+  f4 a[8], b[8];
+  read(a, 0);
+  for (int i = 0; i < np / 4; i += 16) {
+    read(b, i + 8);
+    add(a);
+    read(a, i + 16);
+    add(b);
+  }
+  return ss;
+}
+
 // LDS: per row the quantized activation blocks (XB bytes each), Q4_K's sums of
 // 32 elements and the blocks' d; the block terms [matrix][row][block][16][NT];
-// the class sums [matrix][row][16][9]
+// the class sums [matrix][row][16][9]; with a norm, the squares of each row
+// (sq_stride floats) and its rms
 template <int FMT>
 struct Lds {
   static constexpr int XB = FMT == FMT_Q4K ? 256 : 512;
@@ -66,41 +100,77 @@ struct Lds {
   int nb;
   char* x;
   int* bs;
-  float *d, *t, *s;
+  float *d, *t, *s, *sq, *rms;
   __device__ Lds(char* base, int nb_, int rb, int nm) : nb(nb_) {
     x = base;
     t = reinterpret_cast<float*>(x + (size_t)rb * nb * XB);
     s = t + (size_t)nm * rb * nb * kRows * NT;
     bs = reinterpret_cast<int*>(s + nm * rb * kRows * 9);
     d = reinterpret_cast<float*>(bs + (size_t)rb * nb * NS);
+    rms = d + (size_t)rb * nb;
+    sq = reinterpret_cast<float*>(((uintptr_t)(rms + rb) + 15) & ~(uintptr_t)15);
   }
-  static size_t bytes(int nb, int rb, int nm) {
-    return (size_t)rb * nb * (XB + NS * 4 + 4) + (size_t)nm * rb * kRows * (nb * NT + 9) * 4;
+  static size_t bytes(int nb, int rb, int nm, int norm_n = 0) {
+    return (size_t)rb * nb * (XB + NS * 4 + 4) + (size_t)nm * rb * kRows * (nb * NT + 9) * 4 +
+           (norm_n ? (size_t)rb * (sq_stride(norm_n) + 1) * 4 + 16 : 0);
   }
   __device__ float* term(int m, int rb, int r, int b, int row) const {
     return t + ((((size_t)m * rb + r) * nb + b) * kRows + row) * NT;
   }
 };
 
+// Eight consecutive elements of a row of n (zeros past its end).
+__device__ inline void load8(const float* p, int left, float (&v)[8]) {
+  if (left >= 8 && (((uintptr_t)p) & 15) == 0) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const f4 w = reinterpret_cast<const f4*>(p)[i];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[4 * i + k] = w[k];
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = i < left ? p[i] : 0.0f;
+  }
+}
+
 // BlockQ8K::from_float of the launch's rows, the whole workgroup; half a wave
-// per block.
-template <int FMT>
-__device__ void quantize(const float* __restrict__ x, int ldx, int rows, int n_in, const Lds<FMT>& L) {
+// per block. NORM: of x / rms * nw, rms from the squares' left-to-right sum
+// (candle's rms_norm, as rmsnorm_ordered_kernel).
+template <int FMT, bool NORM>
+__device__ void quantize(const float* __restrict__ x, int ldx, int rows, int n_in, const float* __restrict__ nw,
+                         float eps, const Lds<FMT>& L) {
   const int t = threadIdx.x & 31, hi = threadIdx.x & 32, units = rows * L.nb;
-  for (int un = threadIdx.x >> 5; un < units; un += blockDim.x >> 5) {
-    const int r = un / L.nb, b = un - r * L.nb, e0 = b * 256 + 8 * t;
-    const float* xr = x + (size_t)r * ldx + e0;
-    float v[8];
-    if (e0 + 8 <= n_in && (((uintptr_t)xr) & 15) == 0) {
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const f4 w = reinterpret_cast<const f4*>(xr)[i];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) v[4 * i + k] = w[k];
+  float v[8], wv[8];
+  auto fetch = [&](int un) {
+    const int r = un / L.nb, e0 = (un - r * L.nb) * 256 + 8 * t;
+    load8(x + (size_t)r * ldx + e0, n_in - e0, v);
+    if constexpr (NORM) load8(nw + e0, n_in - e0, wv);
+  };
+  const int first = threadIdx.x >> 5, step = blockDim.x >> 5;
+  if constexpr (NORM) {
+    const int ld = sq_stride(n_in), np = ld - 64;
+    for (int un = first; un < units; un += step) {
+      const int r = un / L.nb, e = (un - r * L.nb) * 256 + 8 * t;
+      fetch(un);
+      if (e < np) {
+        f4* q = reinterpret_cast<f4*>(L.sq + r * ld + e);
+        q[0] = f4{v[0] * v[0], v[1] * v[1], v[2] * v[2], v[3] * v[3]};
+        q[1] = f4{v[4] * v[4], v[5] * v[5], v[6] * v[6], v[7] * v[7]};
       }
-    } else {
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < rows)
+      L.rms[threadIdx.x] = sqrtf(ordered_sum(L.sq + threadIdx.x * ld, np) / (float)n_in + eps);
+    __syncthreads();
+  }
+  for (int un = first; un < units; un += step) {
+    const int r = un / L.nb, b = un - r * L.nb;
+    if (!NORM || units > step) fetch(un);  // else still in registers
+    if constexpr (NORM) {
+      const float m = L.rms[r];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = e0 + i < n_in ? xr[i] : 0.0f;
+      for (int i = 0; i < 8; ++i) v[i] = v[i] / m * wv[i];
     }
     float amax = 0.0f, mx = 0.0f;
 #pragma unroll
@@ -267,7 +337,7 @@ struct Raw<FMT_Q6K> {
 
 // The tiles of one matrix (two for SwiGLU) that this workgroup owns: block
 // terms, the ordered sums, the epilogue. rb: row capacity of the LDS layout.
-template <int FMT, int EPI>
+template <int FMT, int EPI, bool NORM>
 __device__ void run_tiles(const GemvArgs& a, int first, int ntiles, int stride, int rows, int rb, char* lds) {
   constexpr int NM = EPI == EPI_SWIGLU ? 2 : 1, NC = Lds<FMT>::NC;
   const int nb = a.nsb, units = NM * nb, nw = blockDim.x >> 6, wv = threadIdx.x >> 6;
@@ -280,7 +350,7 @@ __device__ void run_tiles(const GemvArgs& a, int first, int ntiles, int stride, 
   // a wave without a block of its own loads (and drops) the last one
   Raw<FMT> cur, nxt;
   load(cur, first, min(wv, units - 1));
-  quantize<FMT>(reinterpret_cast<const float*>(a.x), a.ldx, rows, a.n_in, L);
+  quantize<FMT, NORM>(reinterpret_cast<const float*>(a.x), a.ldx, rows, a.n_in, a.norm_w, a.norm_eps, L);
   __syncthreads();
   for (int tile = first; tile < ntiles; tile += stride) {
     for (int unit = wv; unit < units; unit += nw) {
@@ -333,20 +403,20 @@ __device__ void run_tiles(const GemvArgs& a, int first, int ntiles, int stride, 
   }
 }
 
-template <int FMT, int EPI>
+template <int FMT, int EPI, bool NORM>
 __global__ __launch_bounds__(64 * kMaxWaves) void q8k_kernel(GemvArgs a, int ntiles, int rows, int rb) {
   extern __shared__ __attribute__((aligned(16))) char dsm[];
-  run_tiles<FMT, EPI>(a, blockIdx.x, ntiles, gridDim.x, rows, rb, dsm);
+  run_tiles<FMT, EPI, NORM>(a, blockIdx.x, ntiles, gridDim.x, rows, rb, dsm);
 }
 
 // Two matrices of one input: workgroups below split take tiles of a, the rest
 // of b, each quantizing the rows in its own format's layout.
-template <int FMT, int FMT2>
+template <int FMT, int FMT2, bool NORM>
 __global__ __launch_bounds__(64 * kMaxWaves) void q8k_pair_kernel(GemvArgs a, GemvArgs b, int split, int rows, int rb) {
   extern __shared__ __attribute__((aligned(16))) char dsm[];
   const int id = blockIdx.x;
-  if (id < split) run_tiles<FMT, EPI_STORE>(a, id, id + 1, 1, rows, rb, dsm);
-  else run_tiles<FMT2, EPI_STORE>(b, id - split, id - split + 1, 1, rows, rb, dsm);
+  if (id < split) run_tiles<FMT, EPI_STORE, NORM>(a, id, id + 1, 1, rows, rb, dsm);
+  else run_tiles<FMT2, EPI_STORE, NORM>(b, id - split, id - split + 1, 1, rows, rb, dsm);
 }
 
 constexpr size_t kLdsMax = 160 * 1024;
@@ -375,40 +445,45 @@ void advance(GemvArgs& a, int rows) {
   if (a.res) a.res += (size_t)rows * a.ldres;
 }
 
-template <int FMT, int EPI>
+template <int FMT, int EPI, bool NORM>
 void launch(GemvArgs a, int nrows, hipStream_t s) {
   constexpr int NM = EPI == EPI_SWIGLU ? 2 : 1;
+  auto need = [&](int rb) { return Lds<FMT>::bytes(a.nsb, rb, NM, NORM ? a.n_in : 0); };
   // wide rows: one row per launch where the rows' terms do not fit together
-  const int rb = Lds<FMT>::bytes(a.nsb, nrows, NM) <= kLdsMax ? nrows : 1;
-  const size_t lds = Lds<FMT>::bytes(a.nsb, rb, NM);
+  const int rb = need(nrows) <= kLdsMax ? nrows : 1;
+  const size_t lds = need(rb);
   PGD_CHECK(lds <= kLdsMax, kErrShape, "activation rows too wide for the quantized-activation GEMV");
   if (lds > 64 * 1024) {
-    static const bool ok = (allow_lds(&q8k_kernel<FMT, EPI>), true);
+    static const bool ok = (allow_lds(&q8k_kernel<FMT, EPI, NORM>), true);
     (void)ok;
   }
   const int tiles = tiles_of(a.n_out), nw = waves_of(NM * a.nsb);
   for (int r0 = 0; r0 < nrows; r0 += rb) {
     const int rows = min(rb, nrows - r0);
-    hipLaunchKernelGGL((q8k_kernel<FMT, EPI>), dim3(min(tiles, kMaxGroups)), dim3(64 * nw), lds, s, a, tiles, rows, rb);
+    hipLaunchKernelGGL((q8k_kernel<FMT, EPI, NORM>), dim3(min(tiles, kMaxGroups)), dim3(64 * nw), lds, s, a, tiles,
+                       rows, rb);
     PGD_HIP(hipGetLastError());
     advance(a, rows);
   }
 }
 
-template <int FMT, int FMT2>
+template <int FMT, int FMT2, bool NORM>
 void launch_pair(GemvArgs a, GemvArgs b, int nrows, hipStream_t s) {
-  auto need = [&](int rb) { return std::max(Lds<FMT>::bytes(a.nsb, rb, 1), Lds<FMT2>::bytes(a.nsb, rb, 1)); };
+  auto need = [&](int rb) {
+    const int n = NORM ? a.n_in : 0;
+    return std::max(Lds<FMT>::bytes(a.nsb, rb, 1, n), Lds<FMT2>::bytes(a.nsb, rb, 1, n));
+  };
   const int rb = need(nrows) <= kLdsMax ? nrows : 1;
   const size_t lds = need(rb);
   PGD_CHECK(lds <= kLdsMax, kErrShape, "activation rows too wide for the quantized-activation GEMV");
   if (lds > 64 * 1024) {
-    static const bool ok = (allow_lds(&q8k_pair_kernel<FMT, FMT2>), true);
+    static const bool ok = (allow_lds(&q8k_pair_kernel<FMT, FMT2, NORM>), true);
     (void)ok;
   }
   const int ta = tiles_of(a.n_out), tb = tiles_of(b.n_out), nw = waves_of(a.nsb);
   for (int r0 = 0; r0 < nrows; r0 += rb) {
     const int rows = min(rb, nrows - r0);
-    hipLaunchKernelGGL((q8k_pair_kernel<FMT, FMT2>), dim3(ta + tb), dim3(64 * nw), lds, s, a, b, ta, rows, rb);
+    hipLaunchKernelGGL((q8k_pair_kernel<FMT, FMT2, NORM>), dim3(ta + tb), dim3(64 * nw), lds, s, a, b, ta, rows, rb);
     PGD_HIP(hipGetLastError());
     advance(a, rows);
     advance(b, rows);
@@ -417,9 +492,20 @@ void launch_pair(GemvArgs a, GemvArgs b, int nrows, hipStream_t s) {
 
 template <int FMT>
 void run_epi(const GemvArgs& a, int nrows, int epi, hipStream_t s) {
-  if (epi == EPI_SWIGLU) launch<FMT, EPI_SWIGLU>(a, nrows, s);
-  else if (epi == EPI_RES) launch<FMT, EPI_RES>(a, nrows, s);
-  else launch<FMT, EPI_STORE>(a, nrows, s);
+  if (epi == EPI_SWIGLU) {
+    if (a.norm_w) launch<FMT, EPI_SWIGLU, true>(a, nrows, s);
+    else launch<FMT, EPI_SWIGLU, false>(a, nrows, s);
+  } else if (epi == EPI_RES) {
+    launch<FMT, EPI_RES, false>(a, nrows, s);
+  } else {
+    launch<FMT, EPI_STORE, false>(a, nrows, s);
+  }
+}
+
+template <int FMT, int FMT2>
+void run_pair(const GemvArgs& a, const GemvArgs& b, int nrows, hipStream_t s) {
+  if (a.norm_w) launch_pair<FMT, FMT2, true>(a, b, nrows, s);
+  else launch_pair<FMT, FMT2, false>(a, b, nrows, s);
 }
 
 }  // namespace
@@ -430,10 +516,15 @@ void run_q8k_gemv(int fmt, const GemvArgs& a, int nrows, int epi, hipStream_t s)
 }
 
 void run_q8k_gemv_pair(int fmt_a, const GemvArgs& a, int fmt_b, const GemvArgs& b, int nrows, hipStream_t s) {
-  if (fmt_a == FMT_Q4K && fmt_b == FMT_Q4K) launch_pair<FMT_Q4K, FMT_Q4K>(a, b, nrows, s);
-  else if (fmt_a == FMT_Q4K) launch_pair<FMT_Q4K, FMT_Q6K>(a, b, nrows, s);
-  else if (fmt_b == FMT_Q4K) launch_pair<FMT_Q6K, FMT_Q4K>(a, b, nrows, s);
-  else launch_pair<FMT_Q6K, FMT_Q6K>(a, b, nrows, s);
+  if (fmt_a == FMT_Q4K && fmt_b == FMT_Q4K) run_pair<FMT_Q4K, FMT_Q4K>(a, b, nrows, s);
+  else if (fmt_a == FMT_Q4K) run_pair<FMT_Q4K, FMT_Q6K>(a, b, nrows, s);
+  else if (fmt_b == FMT_Q4K) run_pair<FMT_Q6K, FMT_Q4K>(a, b, nrows, s);
+  else run_pair<FMT_Q6K, FMT_Q6K>(a, b, nrows, s);
+}
+
+bool q8k_norm_ok(int tiles16, int nsb, int n_in, int nrows, int nm) {
+  return tiles16 <= 512 && n_in <= 8192 &&
+         std::max(Lds<FMT_Q4K>::bytes(nsb, nrows, nm, n_in), Lds<FMT_Q6K>::bytes(nsb, nrows, nm, n_in)) <= kLdsMax;
 }
 
 }  // namespace gemv

@@ -612,13 +612,13 @@ void step(Model& m, Session* const* sess, const uint32_t* toks, const int* n, in
           ld_q = ld_kv = (int)w.lda;
         }
       } else {
-        rmsnorm_rows(w.x, H, nullptr, rows, H, L.in_norm, eps, norm_mode, w.xn, H, st);
         // q | k | v side by side in A (q and k from one stacked launch when they share a format)
         float* yv = w.A + m.q_out + m.kv_width;
         if (L.proj.base && m.q8act && qmat_q8act_pairable(L.proj, L.v)) {
-          // stacked q|k and v in one launch (one activation quantization)
-          qmat_gemv_q8act_pair(L.proj, w.A, L.v, yv, w.xn, H, rows, (int)w.lda, st);
+          // stacked q|k and v in one launch (one norm and activation quantization)
+          qmat_gemv_q8act_pair_norm(L.proj, w.A, L.v, yv, w.x, H, L.in_norm, eps, w.xn, rows, (int)w.lda, st);
         } else {
+          rmsnorm_rows(w.x, H, nullptr, rows, H, L.in_norm, eps, norm_mode, w.xn, H, st);
           if (L.proj.base) {
             gemv(L.proj, w.xn, H, rows, w.A, (int)w.lda, nullptr, 0);
           } else {
@@ -710,9 +710,12 @@ void step(Model& m, Session* const* sess, const uint32_t* toks, const int* n, in
           qmat_gemv_a8(L.down, mid, w.x, H, w.x, H, st);
         }
       } else {
-        rmsnorm_rows(w.x, H, nullptr, rows, H, L.post_norm, eps, norm_mode, w.xn, H, st);
-        if (m.q8act) qmat_gemv_swiglu_q8act(L.gate, L.up, w.xn, H, rows, w.G, c.intermediate, st);
-        else qmat_gemv_swiglu(L.gate, L.up, w.xn, H, rows, w.G, c.intermediate, st);
+        if (m.q8act) {
+          qmat_gemv_swiglu_q8act_norm(L.gate, L.up, w.x, H, L.post_norm, eps, w.xn, rows, w.G, c.intermediate, st);
+        } else {
+          rmsnorm_rows(w.x, H, nullptr, rows, H, L.post_norm, eps, norm_mode, w.xn, H, st);
+          qmat_gemv_swiglu(L.gate, L.up, w.xn, H, rows, w.G, c.intermediate, st);
+        }
         gemv(L.down, w.G, c.intermediate, rows, w.x, H, w.x, H);
       }
     }

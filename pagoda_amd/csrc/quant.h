@@ -132,6 +132,14 @@ bool qmat_q8act_pairable(const QMat& a, const QMat& b);
 void qmat_gemv_q8act_pair(const QMat& a, float* ya, const QMat& b, float* yb, const float* x, int ldx, int nrows,
                           int ldy, hipStream_t s);
 
+// The two calls above over rows normed first (rmsnorm_rows mode 2: x / rms * nw,
+// the squares summed left to right): inside the launch where that pays, else
+// through xn (at least nrows rows of stride ldx); the same bits either way.
+void qmat_gemv_swiglu_q8act_norm(const QMat& gate, const QMat& up, const float* x, int ldx, const float* nw, float eps,
+                                 float* xn, int nrows, float* mid, int ldm, hipStream_t s);
+void qmat_gemv_q8act_pair_norm(const QMat& a, float* ya, const QMat& b, float* yb, const float* x, int ldx,
+                               const float* nw, float eps, float* xn, int nrows, int ldy, hipStream_t s);
+
 // fused SwiGLU: mid[r, n] = silu(gate.x) * (up.x)
 void qmat_gemv_swiglu(const QMat& gate, const QMat& up, const float* x, int ldx, int nrows, float* mid,
                       int ldm, hipStream_t s);

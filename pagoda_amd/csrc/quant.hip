@@ -8,6 +8,7 @@
 
 #include "common.h"
 #include "gemv_impl.h"
+#include "ops.h"
 #include "quant.h"
 
 namespace pgd {
@@ -682,8 +683,11 @@ bool qmat_q8act_pairable(const QMat& a, const QMat& b) {
   return a.n_in == b.n_in && gemv::q8act_pair_ok(a.fmt, b.fmt);
 }
 
-void qmat_gemv_q8act_pair(const QMat& a, float* ya, const QMat& b, float* yb, const float* x, int ldx, int nrows,
-                          int ldy, hipStream_t s) {
+namespace {
+int tiles16(const QMat& m) { return (m.n_out + 15) / 16; }
+
+void q8act_pair(const QMat& a, float* ya, const QMat& b, float* yb, const float* x, int ldx, const float* nw, float eps,
+                int nrows, int ldy, hipStream_t s) {
   PGD_CHECK(nrows >= 0 && ldx >= a.n_in && ldy >= a.n_out && ldy >= b.n_out, kErrShape, "gemv rows / strides");
   if (nrows == 0) return;
   GemvArgs ga = make_args(a), gb = make_args(b);
@@ -692,11 +696,13 @@ void qmat_gemv_q8act_pair(const QMat& a, float* ya, const QMat& b, float* yb, co
   ga.y = ya;
   gb.y = yb;
   ga.ldy = gb.ldy = ldy;
+  ga.norm_w = gb.norm_w = nw;
+  ga.norm_eps = gb.norm_eps = eps;
   run_q8act_pair(a.fmt, ga, b.fmt, gb, nrows, s);
 }
 
-void qmat_gemv_swiglu_q8act(const QMat& gate, const QMat& up, const float* x, int ldx, int nrows, float* mid, int ldm,
-                            hipStream_t s) {
+void q8act_swiglu(const QMat& gate, const QMat& up, const float* x, int ldx, const float* nw, float eps, int nrows,
+                  float* mid, int ldm, hipStream_t s) {
   PGD_CHECK(gate.fmt == up.fmt && gate.n_out == up.n_out && gate.n_in == up.n_in, kErrShape,
             "swiglu gate/up shapes differ");
   PGD_CHECK(nrows >= 0 && ldx >= gate.n_in, kErrShape, "gemv rows / ldx");
@@ -710,7 +716,36 @@ void qmat_gemv_swiglu_q8act(const QMat& gate, const QMat& up, const float* x, in
   a.ldx = ldx;
   a.y = mid;
   a.ldy = ldm;
+  a.norm_w = nw;
+  a.norm_eps = eps;
   run_q8act(gate.fmt, a, nrows, EPI_SWIGLU, s);
+}
+}  // namespace
+
+void qmat_gemv_q8act_pair(const QMat& a, float* ya, const QMat& b, float* yb, const float* x, int ldx, int nrows,
+                          int ldy, hipStream_t s) {
+  q8act_pair(a, ya, b, yb, x, ldx, nullptr, 0.0f, nrows, ldy, s);
+}
+
+void qmat_gemv_q8act_pair_norm(const QMat& a, float* ya, const QMat& b, float* yb, const float* x, int ldx,
+                               const float* nw, float eps, float* xn, int nrows, int ldy, hipStream_t s) {
+  if (gemv::q8act_norm_fused(a.fmt, tiles16(a) + tiles16(b), a.nsb, a.n_in, nrows, 1))
+    return q8act_pair(a, ya, b, yb, x, ldx, nw, eps, nrows, ldy, s);
+  rmsnorm_rows(x, ldx, nullptr, nrows, a.n_in, nw, eps, 2, xn, ldx, s);
+  q8act_pair(a, ya, b, yb, xn, ldx, nullptr, 0.0f, nrows, ldy, s);
+}
+
+void qmat_gemv_swiglu_q8act(const QMat& gate, const QMat& up, const float* x, int ldx, int nrows, float* mid, int ldm,
+                            hipStream_t s) {
+  q8act_swiglu(gate, up, x, ldx, nullptr, 0.0f, nrows, mid, ldm, s);
+}
+
+void qmat_gemv_swiglu_q8act_norm(const QMat& gate, const QMat& up, const float* x, int ldx, const float* nw, float eps,
+                                 float* xn, int nrows, float* mid, int ldm, hipStream_t s) {
+  if (gemv::q8act_norm_fused(gate.fmt, tiles16(gate), gate.nsb, gate.n_in, nrows, 2))
+    return q8act_swiglu(gate, up, x, ldx, nw, eps, nrows, mid, ldm, s);
+  rmsnorm_rows(x, ldx, nullptr, nrows, gate.n_in, nw, eps, 2, xn, ldx, s);
+  q8act_swiglu(gate, up, xn, ldx, nullptr, 0.0f, nrows, mid, ldm, s);
 }
 
 void qmat_gemv_a8(const QMat& m, const A8Act& act, float* y, int ldy, const float* res, int ldres, hipStream_t s) {

@@ -121,6 +121,31 @@ def test_qwen2_cpu_arithmetic_bitwise_every_head_dim(dev, head_dim):
     m.free()
 
 
+@pytest.mark.parametrize("hidden,heads,kv_heads,inter", [(256, 4, 2, 512), (320, 5, 1, 512), (1216, 19, 1, 2112),
+                                                         (2304, 36, 4, 8448)])
+def test_qwen2_batch_sizes_bitwise_equal(dev, hidden, heads, kv_heads, inter):
+    """A decode row's logits have the same bits in every kernel the batch size
+    selects (CPU-order arithmetic): the RMSNorm inside the projection launches
+    (1, 4 and 6 rows; row widths of whole and partial blocks and rounds), as a
+    launch of its own before the matrix-core GEMM (7 and 17 rows), and, for the
+    widest feed-forward matrix here, before the few-row GEMV."""
+    from pagoda_amd.engine import Model
+
+    cfg = small2(hidden=hidden, heads=heads, kv_heads=kv_heads, intermediate=inter, n_layers=2)
+    m = Model.synth(dev, cfg, 5)
+    rng = np.random.default_rng(hidden)
+    root = m.new_session()
+    root.forward(rng.integers(0, cfg.vocab, 3))
+    toks = rng.integers(0, cfg.vocab, 17)
+    ref = [root.fork().forward([t]) for t in toks]
+    for n in (2, 4, 6, 7, 17):
+        _, got = m.step_ragged([root.fork() for _ in range(n)], [[t] for t in toks[:n]], want_logits=True)
+        for i in range(n):
+            np.testing.assert_array_equal(got[i].view(np.uint32), ref[i].view(np.uint32), err_msg=f"{n} rows, row {i}")
+    root.free()
+    m.free()
+
+
 @pytest.mark.parametrize("which", ["m35", "m2"])
 def test_ragged_batch_bitwise_equals_serial(which, request):
     """Batched step == per-session forwards (pagoda/tests/batch_tests.rs:217-242).
