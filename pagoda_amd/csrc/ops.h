@@ -56,6 +56,7 @@ struct GdnParams {
   // form before their gated norm, [rows, v_heads * v_dim] (null: step kernel only)
   float* o_raw;
   int o_rows;  // rows of o_raw (rows past it are not written or read)
+  int chunk_cap;  // chunks its scratch holds
 };
 
 // Gated-DeltaNet recurrence over each sequence's rows in order

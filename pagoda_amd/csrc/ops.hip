@@ -1,5 +1,7 @@
 // ops.hip — RMSNorm, causal conv step, Gated-DeltaNet recurrence, q/k/v
 // preparation with paged KV writes and argmax (attention: attn.hip).
+#include <climits>
+
 #include "common.h"
 #include "ops.h"
 #include "gemv_impl.h"
@@ -219,6 +221,24 @@ __device__ inline float softplus_f(float x) {
   return logf(1.0f + expf(x));
 }
 
+__device__ inline int gdn_chunks(int n) { return n < kGdnLongRows ? 0 : (n + kGdnChunk - 1) / kGdnChunk; }
+
+// Chunks of the long sequences are numbered in sequence order. The number of
+// sequence s's first one, or -1 when its chunks do not all fit below cap (a
+// caller's rows bound was too small for its counts: gdn_kernel's then). Whole
+// waves call it.
+__device__ inline int gdn_chunk_base(const int* row_count, int s, int cap) {
+  int base = 0;
+  for (int j0 = 0; j0 < s; j0 += 64) {
+    const int j = j0 + (threadIdx.x & 63);
+    int c = j < s ? gdn_chunks(row_count[j]) : 0;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) c += __shfl_xor(c, o, 64);
+    base += c;
+  }
+  return base + gdn_chunks(row_count[s]) <= cap ? base : -1;
+}
+
 constexpr int kGdnRowGroups = 16;
 
 template <int RG>
@@ -233,6 +253,10 @@ __global__ __launch_bounds__(32 * RG) void gdn_kernel(GdnParams p, const int* ro
   const int repeat = p.v_heads / p.k_heads;
   const int kh = h / repeat;
   const int key_dim = p.k_heads * D;
+  const int r0 = row_start[s], n = row_count[s];
+  // the chunkwise kernels' (unless their scratch does not hold the sequence)
+  if (p.o_raw && n >= kGdnLongRows && gdn_chunk_base(row_count, s, p.chunk_cap) >= 0) return;
+  const int row_end = p.o_raw ? p.o_rows : INT_MAX;  // a prefill's rows past its bound are not written
   float* st = p.state_base[s] + p.state_off + (size_t)h * D * D;
   float S[RPT][4];
 #pragma unroll
@@ -245,8 +269,6 @@ __global__ __launch_bounds__(32 * RG) void gdn_kernel(GdnParams p, const int* ro
   }
   const float a_log = p.a_log[h], dtb = p.dt_bias[h];
   const float qscale = sqrtf((float)D);
-  const int r0 = row_start[s], n = row_count[s];
-  if (p.o_raw && n >= kGdnLongRows) return;  // gdn_chunk_kernel's
   // the gate input z and the norm weight are loaded with the step's other
   // inputs, not after the reductions that need them
   const float nw = tid < D ? p.norm[tid] : 0.0f;
@@ -338,11 +360,11 @@ __global__ __launch_bounds__(32 * RG) void gdn_kernel(GdnParams p, const int* ro
     if (tid < D) {
       const float inv = 1.0f / sqrtf((part[0] + part[1]) / (float)D + 1e-6f);
       const float val = o * inv * nw * (zg / (1.0f + expf(-zg)));
-      if (p.out) p.out[(size_t)row * p.ld_out + h * D + tid] = val;
+      if (p.out && row < row_end) p.out[(size_t)row * p.ld_out + h * D + tid] = val;
       obuf[tid] = val;
     }
     __syncthreads();
-    if (p.act.XA && tid < D / 16) {
+    if (p.act.XA && tid < D / 16 && row < row_end) {
       // the head's 128 outputs are two whole groups of the out projection's input
       float v[16];
 #pragma unroll
@@ -361,284 +383,433 @@ __global__ __launch_bounds__(32 * RG) void gdn_kernel(GdnParams p, const int* ro
 // chunk of m tokens from state S0, with G_t the running sum of the log decay
 // g from the chunk start, gamma_t = exp(G_t), and the sequential recurrence
 // S_t = a_t S_{t-1} + k_t d_t^T, d_t = beta_t (v_t - (a_t S_{t-1})^T k_t):
-//   d_t = U_t - sum_{i<t} L_ti d_i,  U_t = beta_t (v_t - gamma_t S0^T k_t),
-//                                    L_ti = beta_t exp(G_t - G_i) (k_t . k_i)
-//   o_t = gamma_t S0^T q_t + sum_{i<=t} exp(G_t - G_i) (q_t . k_i) d_i
+//   d = T U,  T = (I + L)^-1,  U_t = beta_t (v_t - gamma_t S0^T k_t),
+//                              L_ti = beta_t exp(G_t - G_i) (k_t . k_i), i < t
+//   o_t = gamma_t S0^T q_t + sum_{i<=t} B_ti d_i,  B_ti = exp(G_t - G_i) (q_t . k_i)
 //   S_m = gamma_m S0 + sum_i exp(G_m - G_i) k_i d_i^T
-// (every decay factor exp(G_t - G_i) with t >= i is at most 1). A column of S
-// (one value dimension) evolves on its own, so a head's 128 columns are split
-// over kGdnColGroups workgroups (grid x = value head * groups + group), each
-// holding its 128 x 32 slice of S in LDS and repeating the 32 x 32 token
-// products. q and k are L2 normalized per token as in the step kernel and
-// kept transposed ([k index][token]) for float4 reads in the register-blocked
-// products. The recurrence outputs go to o_raw; gdn_norm_kernel applies the
-// gated RMSNorm.
-constexpr int kGdnColGroups = 4;
-constexpr int kGdnCols = 128 / kGdnColGroups;                  // 32 columns of S per workgroup
-constexpr int kGdnCP = kGdnCols + 4, kGdnTP = kGdnChunk + 4;  // padded LDS row strides
-constexpr size_t kGdnChunkLds =
-    (size_t)(3 * 128 * kGdnTP + 2 * kGdnChunk * kGdnCP + 2 * kGdnChunk * kGdnTP + 2 * kGdnChunk) * sizeof(float);
+// (every decay factor exp(G_t - G_i) with t >= i is at most 1). T and B do not
+// depend on the state, so the chunks of a sequence are only serial in the
+// products with S. Two kernels:
+//   gdn_prep_kernel, one workgroup per (chunk, key head), every chunk at once:
+//     the token norms, K K^T and Q K^T, and per value head of the key head the
+//     decays, B and T (16 x 16 diagonal blocks by forward substitution);
+//   gdn_scan_kernel, one workgroup per (value head, 16 columns of S, sequence),
+//     serial over the chunks. A column of S evolves on its own. Wave w keeps S
+//     rows 32 w .. 32 w + 31 in registers (8 per lane): a 16x16 tile of the
+//     fp32 MFMA's result is laid out exactly as the next one's B operand, so S,
+//     W = K S0, U and d never leave them. Per chunk: each wave's part of K S0
+//     and Q S0 over its 32 rows (32 MFMAs), one exchange of the parts through
+//     LDS (the only barrier), then d = T U on every wave (12 MFMAs), B d on two
+//     of them, and the wave's S rows (16 MFMAs); q, k and v of the next chunk
+//     load meanwhile, k passes through wave-private LDS for its transpose.
+// The outputs go to o_raw; gdn_norm_kernel applies the gated RMSNorm. Bound:
+// the chain of one chunk, 68 fp32 MFMAs (0.9 us) and the exchange between
+// them. Measured for one sequence of 1500 rows and 32 value heads: prep 17 us,
+// scan 120 us (2.6 us a chunk; 180 us for two such sequences), norm 16 us; for
+// prompts of 211, 562 and 1500 rows 790 -> 205 us against one kernel that
+// repeated the token products and the triangular solve in every column group,
+// inside the serial loop (15.5 us a chunk).
+constexpr int kGdnScanCols = 16;
+constexpr int kGdnHeadFloats = 2 * kGdnChunk * kGdnChunk + 4 * kGdnChunk;  // T | B | beta | gamma | exp(G_m - G) | gamma_m
+constexpr int kGdnKeyFloats = 2 * kGdnChunk;                              // 1 / |k| | 1 / (|q| sqrt(128))
 
-__global__ __launch_bounds__(256) void gdn_chunk_kernel(GdnParams p, const int* row_start, const int* row_count) {
-  constexpr int D = 128, C = kGdnChunk, NCOL = kGdnCols, CP = kGdnCP, TP = kGdnTP;
-  static_assert(C == 32 && NCOL == 32 && CP == TP, "thread mappings assume 32 tokens x 32 columns");
-  extern __shared__ __attribute__((aligned(16))) float gsm[];
-  float* S = gsm;            // [D][CP]  this group's columns of the state (k index major)
-  float* KT = S + D * CP;    // [D][TP]  normalized k, transposed
-  float* QT = KT + D * TP;   // [D][TP]  normalized, scaled q, transposed
-  float* Uc = QT + D * TP;   // [C][CP]  v, then U, then exp(G_m - G_i) d_i
-  float* Zc = Uc + C * CP;   // [C][CP]  gamma_t S0^T q_t
-  float* Lm = Zc + C * CP;   // [C][TP]
-  float* Bm = Lm + C * TP;   // [C][TP]
-  float* Gs = Bm + C * TP;   // [C] running log decay
-  float* Bs = Gs + C;        // [C] beta
-  const int h = blockIdx.x / kGdnColGroups, col0 = (blockIdx.x % kGdnColGroups) * NCOL;
-  const int s = blockIdx.y, tid = threadIdx.x;
+// The sequence and place in it of chunk g; false past the last.
+__device__ inline bool gdn_find_chunk(const int* row_count, int nseq, int cap, int g, int& s, int& c) {
+  const int lane = threadIdx.x & 63;
+  int base = 0;
+  for (int j0 = 0; j0 < nseq; j0 += 64) {
+    const int own = j0 + lane < nseq ? gdn_chunks(row_count[j0 + lane]) : 0;
+    int incl = own;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += y;
+    }
+    const uint64_t hit = __ballot(base + incl > g);
+    if (hit) {
+      const int l = __builtin_ctzll(hit);
+      const int end = base + __shfl(incl, l, 64);
+      s = j0 + l;
+      c = g - (end - __shfl(own, l, 64));
+      return end <= cap;
+    }
+    base += __shfl(incl, 63, 64);
+  }
+  return false;
+}
+
+__global__ __launch_bounds__(256, 4) void gdn_prep_kernel(GdnParams p, const int* row_start, const int* row_count,
+                                                       int nseq, int cap, float* __restrict__ head_out,
+                                                       float* __restrict__ key_out) {
+  constexpr int D = 128, C = kGdnChunk, LD = C + 4;
+  static_assert(C == 32, "two 16-token tiles");
+  __shared__ __attribute__((aligned(16))) f4 part[4 * 6 * 64];  // K K^T and Q K^T tiles of each wave's k range; then L
+  __shared__ float kk[C * LD], qk[C * LD];
+  __shared__ float red[4][2][C];
+  const int g = blockIdx.x, kh = blockIdx.y, tid = threadIdx.x;
+  const int lane = tid & 63, w = tid >> 6, lr = lane & 15, lk = lane >> 4;
+  int s, ci;
+  if (!gdn_find_chunk(row_count, nseq, cap, g, s, ci)) return;
+  const int t0 = ci * C, m = min(C, row_count[s] - t0), r0 = row_start[s] + t0;
+  // token 16 tb + lr, elements 32 w + 16 j + 4 lk ..: both MFMA operands
+  f4 K[2][2], Q[2][2];
+  float sk[2] = {0.f, 0.f}, sq[2] = {0.f, 0.f};
+#pragma unroll
+  for (int tb = 0; tb < 2; ++tb) {
+    const int t = 16 * tb + lr;
+    const float* cv = p.conv_out + (size_t)(r0 + t) * p.ld_conv + kh * D + 32 * w + 4 * lk;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      K[tb][j] = Q[tb][j] = f4{0.f, 0.f, 0.f, 0.f};
+      if (t < m) {
+        Q[tb][j] = *reinterpret_cast<const f4*>(cv + 16 * j);
+        K[tb][j] = *reinterpret_cast<const f4*>(cv + p.k_heads * D + 16 * j);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        sk[tb] += K[tb][j][e] * K[tb][j][e];
+        sq[tb] += Q[tb][j][e] * Q[tb][j][e];
+      }
+    }
+#pragma unroll
+    for (int o = 16; o < 64; o <<= 1) {
+      sk[tb] += __shfl_xor(sk[tb], o, 64);
+      sq[tb] += __shfl_xor(sq[tb], o, 64);
+    }
+    if (lk == 0) {
+      red[w][0][t] = sk[tb];
+      red[w][1][t] = sq[tb];
+    }
+  }
+  __syncthreads();
+  const float qscale = sqrtf((float)D);
+#pragma unroll
+  for (int tb = 0; tb < 2; ++tb) {
+    const int t = 16 * tb + lr;
+    const float ik = 1.0f / sqrtf(((red[0][0][t] + red[1][0][t]) + (red[2][0][t] + red[3][0][t])) + 1e-6f);
+    const float iq = 1.0f / sqrtf(((red[0][1][t] + red[1][1][t]) + (red[2][1][t] + red[3][1][t])) + 1e-6f) / qscale;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      K[tb][j] *= ik;
+      Q[tb][j] *= iq;
+    }
+    if (w == 0 && lk == 0) {
+      float* ko = key_out + ((size_t)g * p.k_heads + kh) * kGdnKeyFloats;
+      ko[t] = ik;
+      ko[C + t] = iq;
+    }
+  }
+  // tiles (0, 0), (1, 0), (1, 1) of both products (the fourth is above the diagonal)
+#pragma unroll
+  for (int x = 0; x < 3; ++x) {
+    const int tb = x > 0, ib = x > 1;
+    f4 a = {0.f, 0.f, 0.f, 0.f}, b = a;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        a = __builtin_amdgcn_mfma_f32_16x16x4f32(K[tb][j][e], K[ib][j][e], a, 0, 0, 0);
+        b = __builtin_amdgcn_mfma_f32_16x16x4f32(Q[tb][j][e], K[ib][j][e], b, 0, 0, 0);
+      }
+    part[(w * 6 + x) * 64 + lane] = a;
+    part[(w * 6 + 3 + x) * 64 + lane] = b;
+  }
+  __syncthreads();
+  for (int i = tid; i < 6 * 64; i += 256) {
+    const f4 v = (part[i] + part[384 + i]) + (part[768 + i] + part[1152 + i]);
+    const int x = (i >> 6) % 3, l = i & 63;
+    float* o = (i < 192 ? kk : qk) + (16 * (x > 0) + 4 * (l >> 4)) * LD + 16 * (x > 1) + (l & 15);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o[r * LD] = v[r];
+  }
+  __syncthreads();
+  // one wave per value head: lanes (half, i) take column i, tokens 16 half ..
+  const int repeat = p.v_heads / p.k_heads, i = lane & 31, half = lane >> 5;
+  float* Lm = reinterpret_cast<float*>(part) + w * C * LD;
+  for (int hh = w; hh < repeat; hh += 4) {
+    const int h = kh * repeat + hh;
+    float G = 0.f, beta = 0.f;
+    if (i < m) {
+      const size_t row = (size_t)(r0 + i) * p.ld_ab + h;
+      G = -expf(p.a_log[h]) * softplus_f(p.a[row] + p.dt_bias[h]);
+      beta = 1.0f / (1.0f + expf(-p.b[row]));
+    }
+#pragma unroll
+    for (int o = 1; o < 32; o <<= 1) {
+      const float y = __shfl_up(G, o, 32);
+      if (i >= o) G += y;
+    }
+    float* out = head_out + ((size_t)g * p.v_heads + h) * kGdnHeadFloats;
+#pragma unroll 4
+    for (int k = 0; k < 16; ++k) {
+      const int t = 16 * half + k;
+      const float gt = __shfl(G, t, 64), bt = __shfl(beta, t, 64);
+      float vl = 0.f, vb = 0.f;
+      if (t < m && i <= t) {
+        const float wd = expf(gt - G);
+        vb = wd * qk[t * LD + i];
+        if (i < t) vl = bt * (wd * kk[t * LD + i]);
+      }
+      Lm[t * LD + i] = vl;
+      out[C * C + t * C + i] = vb;
+    }
+    const float gl = __shfl(G, m - 1, 64);
+    if (half == 0) {
+      float* v = out + 2 * C * C;
+      v[i] = beta;
+      v[C + i] = expf(G);
+      v[2 * C + i] = i < m ? expf(gl - G) : 0.f;
+      v[3 * C + i] = expf(gl);
+    }
+    // T = [[X, 0], [-Y L10 X, Y]], X and Y the inverses of the two diagonal
+    // blocks of I + L: lanes 16 b + j take column j of block b, forward
+    // substitution against the unit vector
+    const int bo = 16 * ((lane >> 4) & 1);
+    float x[16];
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+      float acc = t == lr ? 1.0f : 0.0f;
+#pragma unroll
+      for (int u = 0; u < t; u += 4) {
+        const f4 l4 = *reinterpret_cast<const f4*>(Lm + (bo + t) * LD + bo + u);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (u + e < t) acc = fmaf(-l4[e], x[u + e], acc);
+      }
+      x[t] = acc;
+    }
+    f4 pr = {0.f, 0.f, 0.f, 0.f}, lo = pr;
+    if (half == 0) {
+      // the diagonal blocks replace L's in LDS
+#pragma unroll
+      for (int t = 0; t < 16; ++t) {
+        Lm[(bo + t) * LD + bo + lr] = x[t];
+        out[(bo + t) * C + bo + lr] = x[t];
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const f4 l10 = *reinterpret_cast<const f4*>(Lm + (16 + lr) * LD + 4 * lk);
+    const f4 yt = *reinterpret_cast<const f4*>(Lm + (16 + lr) * LD + 16 + 4 * lk);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      pr = __builtin_amdgcn_mfma_f32_16x16x4f32(l10[e], Lm[(4 * lk + e) * LD + lr], pr, 0, 0, 0);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) lo = __builtin_amdgcn_mfma_f32_16x16x4f32(yt[e], pr[e], lo, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) out[(16 + 4 * lk + r) * C + lr] = -lo[r];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  }
+}
+
+__global__ __launch_bounds__(256, 3) void gdn_scan_kernel(GdnParams p, const int* row_start, const int* row_count,
+                                                       int cap, const float* __restrict__ head_in,
+                                                       const float* __restrict__ key_in) {
+  constexpr int D = 128, C = kGdnChunk, LD = C + 4, NG = D / kGdnScanCols;
+  __shared__ __attribute__((aligned(16))) f4 part[2][4][4][64];  // [chunk parity][wave][W tiles, Z tiles]
+  __shared__ __attribute__((aligned(16))) float kl[4][C * LD];   // each wave's 32 columns of k
+  // workgroups go to the 8 XCDs round robin: give each XCD whole heads, whose
+  // column groups read the same q and k
+  const int per = p.v_heads * NG / 8, id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  const int h = id / NG, col0 = (id % NG) * kGdnScanCols, s = blockIdx.y;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, lr = lane & 15, lk = lane >> 4;
   const int n = row_count[s];
   if (n < kGdnLongRows) return;
-  const int r0 = row_start[s];
-  const int repeat = p.v_heads / p.k_heads, kh = h / repeat, key_dim = p.k_heads * D;
-  const int ldo = p.v_heads * D;
-  float* st = p.state_base[s] + p.state_off + (size_t)h * D * D + col0;
-  for (int i = tid; i < D * NCOL / 4; i += 256)
-    *reinterpret_cast<float4*>(S + (i >> 3) * CP + (i & 7) * 4) =
-        *reinterpret_cast<const float4*>(st + (size_t)(i >> 3) * D + (i & 7) * 4);
-  const float a_log = p.a_log[h], dtb = p.dt_bias[h];
-  const float qscale = sqrtf((float)D);
-  const int c = tid & (NCOL - 1), tq = tid >> 5;  // column phases: column c, tokens 4 tq ..
-  // a chunk's q, k (token (tid / 32) + 8 jj, elements 4 (tid % 32)..) and v
-  // (token tid / 8, columns 4 (tid % 8)..) in registers, loaded one chunk
-  // ahead so that no chunk waits for its inputs; zeros past the sequence
-  float4 qn[4], kn[4], vn;
-  auto load_chunk = [&](int tc) {
-    const int mc = min(C, n - tc);
+  const int base = gdn_chunk_base(row_count, s, cap);
+  if (base < 0) return;
+  const int r0 = row_start[s], kh = h / (p.v_heads / p.k_heads), ldo = p.v_heads * D;
+  float* st = p.state_base[s] + p.state_off + (size_t)h * D * D + col0 + lr;
+  // S[j][r]: row 32 w + 16 j + 4 lk + r, column col0 + lr
+  f4 S[2];
 #pragma unroll
-    for (int jj = 0; jj < 4; ++jj) {
-      const int t = (tid >> 5) + 8 * jj, e = (tid & 31) * 4;
-      qn[jj] = make_float4(0.f, 0.f, 0.f, 0.f);
-      kn[jj] = qn[jj];
-      if (t < mc) {
-        const float* cv = p.conv_out + (size_t)(r0 + tc + t) * p.ld_conv;
-        qn[jj] = *reinterpret_cast<const float4*>(cv + kh * D + e);
-        kn[jj] = *reinterpret_cast<const float4*>(cv + key_dim + kh * D + e);
-      }
-    }
-    const int t = tid >> 3, e = (tid & 7) * 4;
-    vn = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (t < mc)
-      vn = *reinterpret_cast<const float4*>(p.conv_out + (size_t)(r0 + tc + t) * p.ld_conv + 2 * key_dim + h * D +
-                                            col0 + e);
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S[j][r] = st[(size_t)(32 * w + 16 * j + 4 * lk + r) * D];
+  // A chunk's inputs. Each is loaded for the next chunk as soon as this one is
+  // done with its registers (one set: three workgroups fit a CU); tokens past
+  // the sequence re-read its last row, and their T, B, beta and decay entries
+  // drop them.
+  const int nc = gdn_chunks(n);
+  f4 q[2][2], k[2][2], v[2];  // q, k: token 16 tb + lr; v: token 16 tb + 4 lk + r
+  float iq[2], ik[2];
+  f4 T00, T10, T11, be[2], ga[2], wd[2];
+  float gm;
+  auto head = [&](int c) { return head_in + ((size_t)(base + c) * p.v_heads + h) * kGdnHeadFloats; };
+  // tile (tb, ib) of T or B: row 16 tb + lr, columns 16 ib + 4 lk ..
+  auto tile = [&](const float* a, int tb, int ib) {
+    return *reinterpret_cast<const f4*>(a + (16 * tb + lr) * C + 16 * ib + 4 * lk);
   };
-  load_chunk(0);
-
-  for (int t0 = 0; t0 < n; t0 += C) {
-    const int m = min(C, n - t0);
-    __syncthreads();  // the previous chunk is done with every buffer
-    // q and k of the chunk (zeros past m): 32 lanes per token, 4 elements each
+  const float* qp = p.conv_out + kh * D + 32 * w + 4 * lk;
+  const float* vp = p.conv_out + 2 * p.k_heads * D + h * D + col0 + lr;
+  auto load_qk = [&](int c) {
+    const float* kd = key_in + ((size_t)(base + c) * p.k_heads + kh) * kGdnKeyFloats + lr;
 #pragma unroll
-    for (int jj = 0; jj < 4; ++jj) {
-      const int t = (tid >> 5) + 8 * jj, e = (tid & 31) * 4;
-      const float4 q4 = qn[jj], k4 = kn[jj];
-      float sq = q4.x * q4.x + q4.y * q4.y + q4.z * q4.z + q4.w * q4.w;
-      float sk = k4.x * k4.x + k4.y * k4.y + k4.z * k4.z + k4.w * k4.w;
+    for (int tb = 0; tb < 2; ++tb) {
+      const float* row = qp + (size_t)(r0 + min(c * C + 16 * tb + lr, n - 1)) * p.ld_conv;
 #pragma unroll
-      for (int o = 1; o < 32; o <<= 1) {
-        sq += __shfl_xor(sq, o, 64);
-        sk += __shfl_xor(sk, o, 64);
+      for (int j = 0; j < 2; ++j) {
+        q[tb][j] = *reinterpret_cast<const f4*>(row + 16 * j);
+        k[tb][j] = *reinterpret_cast<const f4*>(row + p.k_heads * D + 16 * j);
       }
-      const float iq = 1.0f / sqrtf(sq + 1e-6f), ik = 1.0f / sqrtf(sk + 1e-6f);
-      QT[(e + 0) * TP + t] = (q4.x * iq) / qscale;
-      QT[(e + 1) * TP + t] = (q4.y * iq) / qscale;
-      QT[(e + 2) * TP + t] = (q4.z * iq) / qscale;
-      QT[(e + 3) * TP + t] = (q4.w * iq) / qscale;
-      KT[(e + 0) * TP + t] = k4.x * ik;
-      KT[(e + 1) * TP + t] = k4.y * ik;
-      KT[(e + 2) * TP + t] = k4.z * ik;
-      KT[(e + 3) * TP + t] = k4.w * ik;
+      ik[tb] = kd[16 * tb];
+      iq[tb] = kd[C + 16 * tb];
     }
-    {
-      // v of this group's columns: token tid / 8, 4 columns
-      const int t = tid >> 3, e = (tid & 7) * 4;
-      *reinterpret_cast<float4*>(Uc + t * CP + e) = vn;
+  };
+  auto load_v = [&](int c) {
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[tb][r] = vp[(size_t)(r0 + min(c * C + 16 * tb + 4 * lk + r, n - 1)) * p.ld_conv];
+  };
+  auto load_head = [&](int c) {
+    const float* hd = head(c);
+    T00 = tile(hd, 0, 0);
+    T10 = tile(hd, 1, 0);
+    T11 = tile(hd, 1, 1);
+    const float* vec = hd + 2 * C * C + 4 * lk;
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb) {
+      be[tb] = *reinterpret_cast<const f4*>(vec + 16 * tb);
+      ga[tb] = *reinterpret_cast<const f4*>(vec + C + 16 * tb);
+      wd[tb] = *reinterpret_cast<const f4*>(vec + 2 * C + 16 * tb);
     }
-    if (t0 + C < n) load_chunk(t0 + C);
-    if (tid < 64) {
-      // decay and beta per token, then the running sum of the log decay
-      float g = 0.f, beta = 0.f;
-      if (tid < m) {
-        const size_t row = (size_t)(r0 + t0 + tid) * p.ld_ab + h;
-        g = -expf(a_log) * softplus_f(p.a[row] + dtb);
-        beta = 1.0f / (1.0f + expf(-p.b[row]));
+    gm = hd[2 * C * C + 3 * C];
+  };
+  const f4 zero = {0.f, 0.f, 0.f, 0.f};
+  load_qk(0);
+  load_v(0);
+  load_head(0);
+  for (int c = 0; c < nc; ++c) {
+    const int m = min(C, n - c * C), next = min(c + 1, nc - 1);
+    f4 b0, b1;
+    if (w < 2) {
+      b0 = tile(head(c) + C * C, w, 0);
+      b1 = tile(head(c) + C * C, 1, 1);
+    }
+    f4 W[2] = {zero, zero}, Z[2] = {zero, zero};
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+#pragma unroll
+      for (int tb = 0; tb < 2; ++tb) {
+        k[tb][j] *= ik[tb];
+        q[tb][j] *= iq[tb];
+        *reinterpret_cast<f4*>(&kl[w][(16 * tb + lr) * LD + 16 * j + 4 * lk]) = k[tb][j];
       }
 #pragma unroll
-      for (int o = 1; o < 32; o <<= 1) {
-        const float y = __shfl_up(g, o, 64);
-        if ((tid & 31) >= o) g += y;
-      }
-      if (tid < C) {
-        Gs[tid] = g;
-        Bs[tid] = beta;
-      }
-    }
-    __syncthreads();
-    // fp32 MFMA tiles (v_mfma_f32_16x16x4_f32): lane l supplies A[row l % 16]
-    // [k l / 16] and B[k l / 16][col l % 16] and holds D[4 (l / 16) + r][l % 16].
-    const int lane = tid & 63, wave = tid >> 6, lr = lane & 15, lk = lane >> 4;
-    {
-      // L (t x i, i < t) and B (i <= t) from K K^T and Q K^T over the 128 k:
-      // waves 0..2 take the three nonzero 16x16 tiles of both, wave 3 writes
-      // the zero tile above the diagonal
-      if (wave < 3) {
-        const int tb = wave == 0 ? 0 : 16, ib = wave == 2 ? 16 : 0;
-        f4 aL = {0.f, 0.f, 0.f, 0.f}, aB = aL;
-#pragma unroll 8
-        for (int k0 = 0; k0 < D; k0 += 4) {
-          const float* kr = KT + (k0 + lk) * TP;
-          const float ki = kr[ib + lr];
-          aL = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[tb + lr], ki, aL, 0, 0, 0);
-          aB = __builtin_amdgcn_mfma_f32_16x16x4f32(QT[(k0 + lk) * TP + tb + lr], ki, aB, 0, 0, 0);
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb) {
+          W[tb] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[tb][j][e], S[j][e], W[tb], 0, 0, 0);
+          Z[tb] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[tb][j][e], S[j][e], Z[tb], 0, 0, 0);
         }
-        const int i = ib + lr;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int t = tb + 4 * lk + r;
-          float vl = 0.f, vb = 0.f;
-          if (t < m && i <= t) {
-            const float w = expf(Gs[t] - Gs[i]);
-            vb = w * aB[r];
-            if (i < t) vl = Bs[t] * (w * aL[r]);
-          }
-          Lm[t * TP + i] = vl;
-          Bm[t * TP + i] = vb;
-        }
-      } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int t = 4 * lk + r, i = 16 + lr;
-          Lm[t * TP + i] = 0.f;
-          Bm[t * TP + i] = 0.f;
-        }
-      }
     }
-    {
-      // W = K S0 and Z = Q S0: wave w takes tokens 16 (w / 2).., columns
-      // 16 (w % 2)..; then U = beta (v - gamma W) and gamma Z
-      const int tb = 16 * (wave >> 1), cb = 16 * (wave & 1);
-      f4 aW = {0.f, 0.f, 0.f, 0.f}, aZ = aW;
-#pragma unroll 8
-      for (int k0 = 0; k0 < D; k0 += 4) {
-        const float sv = S[(k0 + lk) * CP + cb + lr];
-        aW = __builtin_amdgcn_mfma_f32_16x16x4f32(KT[(k0 + lk) * TP + tb + lr], sv, aW, 0, 0, 0);
-        aZ = __builtin_amdgcn_mfma_f32_16x16x4f32(QT[(k0 + lk) * TP + tb + lr], sv, aZ, 0, 0, 0);
-      }
-      const int cc = cb + lr;
+    load_qk(next);
+    __builtin_amdgcn_sched_barrier(0);
+    f4(*pc)[4][64] = part[c & 1];
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb) {
+      pc[w][tb][lane] = W[tb];
+      pc[w][2 + tb][lane] = Z[tb];
+    }
+    __syncthreads();  // (the other parity's parts were read before the previous one)
+    auto whole = [&](int x) { return (pc[0][x][lane] + pc[1][x][lane]) + (pc[2][x][lane] + pc[3][x][lane]); };
+    f4 U[2], d[2] = {zero, zero};
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb) U[tb] = be[tb] * (v[tb] - ga[tb] * whole(tb));
+    load_v(next);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      d[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(T00[e], U[0][e], d[0], 0, 0, 0);
+      d[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(T10[e], U[0][e], d[1], 0, 0, 0);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) d[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(T11[e], U[1][e], d[1], 0, 0, 0);
+    if (w < 2) {
+      // outputs of tokens 16 w ..
+      f4 o = (w ? ga[1] : ga[0]) * whole(2 + w);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o = __builtin_amdgcn_mfma_f32_16x16x4f32(b0[e], d[0][e], o, 0, 0, 0);
+      if (w)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o = __builtin_amdgcn_mfma_f32_16x16x4f32(b1[e], d[1][e], o, 0, 0, 0);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int t = tb + 4 * lk + r;
-        const float gam = expf(Gs[t]), bet = Bs[t];
-        Uc[t * CP + cc] = bet * (Uc[t * CP + cc] - gam * aW[r]);
-        Zc[t * CP + cc] = gam * aZ[r];
+        const int t = 16 * w + 4 * lk + r, row = r0 + c * C + t;
+        if (t < m && row < p.o_rows) p.o_raw[(size_t)row * ldo + h * D + col0 + lr] = o[r];
       }
     }
-    __syncthreads();
-    // d = (I + L)^-1 U for column c, in registers (every thread of the column
-    // solves it; L is zero on and above the diagonal and past the chunk)
-    float d[C];
+    // S = gamma_m S0 + K^T (weighted d)
 #pragma unroll
-    for (int t = 0; t < C; ++t) d[t] = Uc[t * CP + c];
+    for (int tb = 0; tb < 2; ++tb) d[tb] *= wd[tb];
 #pragma unroll
-    for (int t = 1; t < C; ++t) {
-      float acc = d[t];
+    for (int j = 0; j < 2; ++j) S[j] *= gm;
+    load_head(next);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int i = 0; i < t; ++i) acc = fmaf(-Lm[t * TP + i], d[i], acc);
-      d[t] = acc;
-    }
-    // outputs of tokens 4 tq .. for column c: B is zero above the diagonal
+    for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int t = 4 * tq + j;
-      float o = Zc[t * CP + c];
+      for (int e = 0; e < 4; ++e)
 #pragma unroll
-      for (int i4 = 0; i4 < C; i4 += 4) {
-        const float4 b4 = *reinterpret_cast<const float4*>(Bm + t * TP + i4);
-        o = fmaf(b4.x, d[i4], o);
-        o = fmaf(b4.y, d[i4 + 1], o);
-        o = fmaf(b4.z, d[i4 + 2], o);
-        o = fmaf(b4.w, d[i4 + 3], o);
-      }
-      if (t < m && r0 + t0 + t < p.o_rows) p.o_raw[(size_t)(r0 + t0 + t) * ldo + h * D + col0 + c] = o;
-    }
-    const float gl = Gs[m - 1];
-#pragma unroll
-    for (int i = 0; i < C; ++i) d[i] = i < m ? expf(gl - Gs[i]) * d[i] : 0.f;
-    __syncthreads();  // every column's U is read
-    if (tq == 0) {
-#pragma unroll
-      for (int i = 0; i < C; ++i) Uc[i * CP + c] = d[i];
-    }
-    __syncthreads();
-    {
-      // S = gamma_m S0 + K^T (weighted d): wave w takes k rows 32 w .. 32 w + 31
-      // (two 16-row tiles) by both 16-column tiles, 8 MFMA steps over the tokens
-      const float gm = expf(gl);
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-        for (int ct = 0; ct < 2; ++ct) {
-          const int kb = 32 * wave + 16 * kt, cb = 16 * ct;
-          f4 acc;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) acc[r] = gm * S[(kb + 4 * lk + r) * CP + cb + lr];
-#pragma unroll
-          for (int i0 = 0; i0 < C; i0 += 4)
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(KT[(kb + lr) * TP + i0 + lk], Uc[(i0 + lk) * CP + cb + lr], acc,
-                                                       0, 0, 0);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) S[(kb + 4 * lk + r) * CP + cb + lr] = acc[r];
-        }
-    }
+        for (int j = 0; j < 2; ++j)
+          S[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kl[w][(16 * tb + 4 * lk + e) * LD + 16 * j + lr], d[tb][e], S[j],
+                                                      0, 0, 0);
   }
-  __syncthreads();
-  for (int i = tid; i < D * NCOL / 4; i += 256)
-    *reinterpret_cast<float4*>(st + (size_t)(i >> 3) * D + (i & 7) * 4) =
-        *reinterpret_cast<const float4*>(S + (i >> 3) * CP + (i & 7) * 4);
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) st[(size_t)(32 * w + 16 * j + 4 * lk + r) * D] = S[j][r];
 }
 
-// Gated RMSNorm of the chunkwise outputs (rows of long sequences only),
-// exactly the step kernel's tail: out and / or the prepared activations.
-__device__ inline void gdn_norm_row(const GdnParams& p, int row, int h, int tid, float* part, float* obuf) {
+// Gated RMSNorm of the chunkwise outputs (rows of long sequences only), the
+// step kernel's tail: out and / or the prepared activations. grid (row blocks,
+// sequences, groups of four value heads), one wave per head, two elements per
+// lane; a workgroup strides over its sequence's rows, kGdnNormRows loaded at a
+// time. Bound: HBM.
+constexpr int kGdnNormRows = 4;
+__global__ __launch_bounds__(256) void gdn_norm_kernel(GdnParams p, const int* row_start, const int* row_count,
+                                                       int cap) {
   constexpr int D = 128;
-  const float o = p.o_raw[(size_t)row * p.v_heads * D + h * D + tid];
-  const float zg = p.z[(size_t)row * p.ld_z + h * D + tid];
-  const float oss = wave_sum(o * o);
-  if ((tid & 63) == 0) part[tid >> 6] = oss;
-  __syncthreads();
-  const float inv = 1.0f / sqrtf((part[0] + part[1]) / (float)D + 1e-6f);
-  const float val = o * inv * p.norm[tid] * (zg / (1.0f + expf(-zg)));
-  if (p.out) p.out[(size_t)row * p.ld_out + h * D + tid] = val;
-  obuf[tid] = val;
-  __syncthreads();
-  if (p.act.XA && tid < D / 16) {
-    float v[16];
-#pragma unroll
-    for (int e = 0; e < 16; ++e) v[e] = obuf[16 * tid + e];
-    a8act::emit_slice(p.act, row, (h * D + 16 * tid) >> 6, tid & 3, v, true);
-  }
-}
-
-// grid (row blocks, sequence, value head); a workgroup strides over its
-// sequence's rows
-__global__ __launch_bounds__(128) void gdn_norm_kernel(GdnParams p, const int* row_start, const int* row_count) {
-  __shared__ float part[2];
-  __shared__ float obuf[128];
-  const int s = blockIdx.y, h = blockIdx.z, tid = threadIdx.x;
+  __shared__ __attribute__((aligned(16))) float obuf[4][D];
+  const int s = blockIdx.y, w = threadIdx.x >> 6, h = blockIdx.z * 4 + w, lane = threadIdx.x & 63;
   const int n = row_count[s];
-  if (n < kGdnLongRows) return;
+  if (h >= p.v_heads || n < kGdnLongRows || gdn_chunk_base(row_count, s, cap) < 0) return;
+  const float n0 = p.norm[2 * lane], n1 = p.norm[2 * lane + 1];
   // (rows at or past o_rows were never staged: a caller's rows bound was too small)
   const int r0 = row_start[s], t_end = min(n, p.o_rows - r0);
-  for (int t = blockIdx.x; t < t_end; t += gridDim.x) {
-    __syncthreads();  // part and obuf of the previous row are consumed
-    gdn_norm_row(p, r0 + t, h, tid, part, obuf);
+  for (int t0 = blockIdx.x * kGdnNormRows; t0 < t_end; t0 += gridDim.x * kGdnNormRows) {
+    float2 o[kGdnNormRows];
+    float z0[kGdnNormRows], z1[kGdnNormRows];
+#pragma unroll
+    for (int k = 0; k < kGdnNormRows; ++k) {
+      const size_t row = r0 + min(t0 + k, t_end - 1);
+      o[k] = *reinterpret_cast<const float2*>(p.o_raw + row * p.v_heads * D + h * D + 2 * lane);
+      z0[k] = p.z[row * p.ld_z + h * D + 2 * lane];
+      z1[k] = p.z[row * p.ld_z + h * D + 2 * lane + 1];
+    }
+#pragma unroll
+    for (int k = 0; k < kGdnNormRows; ++k) {
+      if (t0 + k >= t_end) break;
+      const int row = r0 + t0 + k;
+      const float inv = 1.0f / sqrtf(wave_sum(o[k].x * o[k].x + o[k].y * o[k].y) / (float)D + 1e-6f);
+      const float v0 = o[k].x * inv * n0 * (z0[k] / (1.0f + expf(-z0[k])));
+      const float v1 = o[k].y * inv * n1 * (z1[k] / (1.0f + expf(-z1[k])));
+      if (p.out) {
+        p.out[(size_t)row * p.ld_out + h * D + 2 * lane] = v0;
+        p.out[(size_t)row * p.ld_out + h * D + 2 * lane + 1] = v1;
+      }
+      if (p.act.XA) {
+        obuf[w][2 * lane] = v0;
+        obuf[w][2 * lane + 1] = v1;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (lane < D / 16) {
+          float v[16];
+#pragma unroll
+          for (int e = 0; e < 16; ++e) v[e] = obuf[w][16 * lane + e];
+          a8act::emit_slice(p.act, row, (h * D + 16 * lane) >> 6, lane & 3, v, true);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      }
+    }
   }
 }
 
@@ -843,26 +1014,32 @@ void gdn_step(const GdnParams& p, SeqMeta meta, int nseq, int rows, int max_rows
   if (nseq <= 0) return;
   const bool chunked = rows > 0 && max_rows >= kGdnLongRows;
   GdnParams q = p;
-  q.o_rows = chunked ? rows : 0;
-  q.o_raw = chunked ? static_cast<float*>(gemv::gemv_scratch(s, (size_t)rows * p.v_heads * 128 * sizeof(float), 7))
-                    : nullptr;
+  q.o_raw = nullptr;
+  q.o_rows = q.chunk_cap = 0;
+  float *head_ws = nullptr, *key_ws = nullptr;
+  if (chunked) {
+    // every long sequence's chunks: at most rows / 32 whole ones and a ragged one each
+    q.o_rows = rows;
+    q.chunk_cap = rows / kGdnChunk + nseq;
+    const size_t o_floats = (size_t)rows * p.v_heads * 128, head_floats = (size_t)q.chunk_cap * p.v_heads * kGdnHeadFloats;
+    const size_t key_floats = (size_t)q.chunk_cap * p.k_heads * kGdnKeyFloats;
+    q.o_raw = static_cast<float*>(gemv::gemv_scratch(s, (o_floats + head_floats + key_floats) * sizeof(float), 7));
+    head_ws = q.o_raw + o_floats;
+    key_ws = head_ws + head_floats;
+  }
   hipLaunchKernelGGL(gdn_kernel<kGdnRowGroups>, dim3(p.v_heads, nseq), dim3(32 * kGdnRowGroups), 0, s, q,
                      meta.row_start, meta.row_count);
   PGD_HIP(hipGetLastError());
   if (!chunked) return;
   PGD_CHECK(p.ld_conv % 4 == 0, kErrShape, "chunked gated delta kernel needs 16-byte aligned conv rows");
-  constexpr size_t lds = kGdnChunkLds;
-  static bool attr = false;
-  if (!attr) {
-    PGD_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gdn_chunk_kernel),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    attr = true;
-  }
-  hipLaunchKernelGGL(gdn_chunk_kernel, dim3(p.v_heads * kGdnColGroups, nseq), dim3(256), lds, s, q, meta.row_start,
-                     meta.row_count);
+  hipLaunchKernelGGL(gdn_prep_kernel, dim3(q.chunk_cap, p.k_heads), dim3(256), 0, s, q, meta.row_start, meta.row_count,
+                     nseq, q.chunk_cap, head_ws, key_ws);
   PGD_HIP(hipGetLastError());
-  hipLaunchKernelGGL(gdn_norm_kernel, dim3(std::min(max_rows, 4096), nseq, p.v_heads), dim3(128), 0, s, q,
-                     meta.row_start, meta.row_count);
+  hipLaunchKernelGGL(gdn_scan_kernel, dim3(p.v_heads * (128 / kGdnScanCols), nseq), dim3(256), 0, s, q, meta.row_start,
+                     meta.row_count, q.chunk_cap, head_ws, key_ws);
+  PGD_HIP(hipGetLastError());
+  hipLaunchKernelGGL(gdn_norm_kernel, dim3(std::min((max_rows + kGdnNormRows - 1) / kGdnNormRows, 4096), nseq, (p.v_heads + 3) / 4), dim3(256), 0, s, q,
+                     meta.row_start, meta.row_count, q.chunk_cap);
   PGD_HIP(hipGetLastError());
 }
 

@@ -1,5 +1,5 @@
-"""The chunkwise form of the gated delta rule that gdn_chunk_kernel (prefill
-of sequences of >= 32 rows) computes, restated in float64 numpy and checked
+"""The chunkwise form of the gated delta rule that gdn_prep_kernel and
+gdn_scan_kernel (prefill of sequences of >= 32 rows) compute, restated in float64 numpy and checked
 against the oracle's per-token recurrence (oracle.c, qwen3_5.rs:1330-1383),
 on the CPU: several chunks, a ragged last chunk, nonzero starting states,
 decay near 1 and near 0. Over a chunk of m tokens from state S0, with G_t the

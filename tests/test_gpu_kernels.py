@@ -148,6 +148,49 @@ def test_gdn_prefill_chunkwise(dev):
         r += n
 
 
+@pytest.mark.parametrize("kh,vh,counts,order", [
+    (16, 32, [32], [0]),                        # one whole chunk
+    (2, 10, [33, 96, 70], [2, 0, 1]),           # five value heads per key head; rows not in sequence order
+    (8, 8, [40, 5, 64] * 23, list(range(69))),  # more sequences than a wave counts at once
+])
+def test_gdn_prefill_chunk_numbering(dev, kh, vh, counts, order):
+    """Where the chunks' scratch is found: sequences laid out in any order, more
+    than 64 of them, head counts of any ratio; and a rows bound below the last
+    sequences, whose rows past it stay unwritten while every state advances."""
+    from pagoda_amd._lib import call
+    import ctypes as C
+
+    rng = np.random.default_rng(sum(counts))
+    rows = sum(counts)
+    starts = np.zeros(len(counts), np.int32)
+    at = 0
+    for s in order:
+        starts[s] = at
+        at += counts[s]
+    conv, a, b, z, a_log, dtb, norm = gdn_inputs(rng, rows, kh, vh)
+    states = (rng.normal(0, 1, (len(counts), vh, 128, 128)) * 0.1).astype(np.float32)
+    d_in = [dev.upload(v) for v in (conv, a, b, z, a_log, dtb, norm)]
+    d_rs, d_rc = dev.upload(starts), dev.upload(np.asarray(counts, np.int32))
+    ref, ref_st = np.zeros((rows, vh * 128), np.float32), states.copy()
+    for s, n in enumerate(counts):
+        sl = slice(int(starts[s]), int(starts[s]) + n)
+        ref[sl] = ora.gdn_step(conv[sl], a[sl], b[sl], z[sl], a_log, dtb, norm, kh, vh, 128, 128, ref_st[s])
+    for bound in (rows, min(32, rows)):
+        sbuf = dev.upload(states)
+        ptrs = dev.upload(np.array([sbuf + s * states[0].nbytes for s in range(len(counts))], np.uint64))
+        d_out = dev.upload(np.full((rows, vh * 128), 7.0, np.float32))
+        call("pgd_gdn_prefill_dev", dev.handle, kh, vh, *[C.c_void_p(q) for q in d_in], C.c_void_p(ptrs),
+             C.c_void_p(d_rs), C.c_void_p(d_rc), len(counts), bound, max(counts), C.c_void_p(d_out))
+        out = dev.download(d_out, (rows, vh * 128), np.float32)
+        assert rel(dev.download(sbuf, states.shape, np.float32), ref_st) < TOL
+        assert rel(out[:bound], ref[:bound]) < TOL
+        assert np.all(out[bound:] == 7.0)
+        for q in (sbuf, ptrs, d_out):
+            dev.free(q)
+    for q in d_in + [d_rs, d_rc]:
+        dev.free(q)
+
+
 def test_gdn_prefill_slow_decay_long(dev):
     """Decay close to 1 (A_log = -8, so a chunk barely forgets) over 200 rows:
     the chunkwise products carry the whole chunk's state instead of rounding
