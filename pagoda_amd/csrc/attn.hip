@@ -35,6 +35,8 @@
 #include <vector>
 
 #include "a8_act.h"
+#include <climits>
+
 #include "common.h"
 #include "gemv_impl.h"
 #include "ops.h"
@@ -589,6 +591,57 @@ void attn_hd(const float* q, const float* gate, float* out, const AttnLayout& L,
 }  // namespace
 
 // ---------------------------------------------------------------------------
+// the rows' metadata to the host
+// ---------------------------------------------------------------------------
+namespace {
+// out (host memory): sequences (highest index + 1), lowest sequence index,
+// seq_of_row, pos_of_row, then the sequences' block tables while they fit in
+// cap ints. Every workgroup finds the range of the indexes for itself and
+// copies its share.
+__global__ __launch_bounds__(256) void attn_meta_kernel(const int* __restrict__ seq, const int* __restrict__ pos,
+                                                        const int* __restrict__ bt, int rows, int max_blocks,
+                                                        int* __restrict__ out, long long cap) {
+  __shared__ int hi[4], lo[4];
+  const int tid = threadIdx.x;
+  int mx = INT_MIN, mn = INT_MAX;
+  for (int r = tid; r < rows; r += 256) {
+    mx = max(mx, seq[r]);
+    mn = min(mn, seq[r]);
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    mx = max(mx, __shfl_xor(mx, o, 64));
+    mn = min(mn, __shfl_xor(mn, o, 64));
+  }
+  if ((tid & 63) == 0) {
+    hi[tid >> 6] = mx;
+    lo[tid >> 6] = mn;
+  }
+  __syncthreads();
+  mx = max(max(hi[0], hi[1]), max(hi[2], hi[3]));
+  mn = min(min(lo[0], lo[1]), min(lo[2], lo[3]));
+  const long long first = (long long)blockIdx.x * 256 + tid, step = (long long)gridDim.x * 256;
+  if (first == 0) {
+    out[0] = mx == INT_MAX ? mx : mx + 1;
+    out[1] = mn;
+  }
+  for (long long i = first; i < rows; i += step) {
+    out[2 + i] = seq[i];
+    out[2 + rows + i] = pos[i];
+  }
+  const long long tables = mn < 0 ? 0 : ((long long)mx + 1) * max_blocks;
+  if (tables <= cap)
+    for (long long i = first; i < tables; i += step) out[2 + 2 * (long long)rows + i] = bt[i];
+}
+}  // namespace
+
+void attn_fetch_meta(const int* seq_of_row, const int* pos_of_row, const int* block_tables, int rows, int max_blocks,
+                     int* out, long long table_cap, hipStream_t s) {
+  hipLaunchKernelGGL(attn_meta_kernel, dim3(32), dim3(256), 0, s, seq_of_row, pos_of_row, block_tables, rows,
+                     max_blocks, out, table_cap);
+  PGD_HIP(hipGetLastError());
+}
+
+// ---------------------------------------------------------------------------
 // host: plan
 // ---------------------------------------------------------------------------
 void build_attn_plan(const int* seq_of_row, const int* pos_of_row, int rows, const int* block_tables,
@@ -597,70 +650,76 @@ void build_attn_plan(const int* seq_of_row, const int* pos_of_row, int rows, con
   // kSplitTiles tiles over the same pages (head_dim 256, attn_split_kernel)
   const int qpi = head_dim == 256 ? 16 * kSplitTiles : 16;
   PGD_CHECK(group > 0 && group <= 64 && block == 16, kErrShape, "attention plan: group <= 64 heads, pages of 16");
+  // A group: the rows whose chunk `chunk` holds the same pages (keys point into
+  // the block tables). A row of the same sequence as the one before it takes
+  // that row's groups for the chunks that are whole in both, without a look-up.
   struct Key {
-    int chunk;
-    std::vector<int> pages;
-    bool operator==(const Key& o) const { return chunk == o.chunk && pages == o.pages; }
+    int chunk, n;
+    const int* pages;
+    bool operator==(const Key& o) const {
+      return chunk == o.chunk && n == o.n && std::equal(pages, pages + n, o.pages);
+    }
   };
   struct KeyHash {
     size_t operator()(const Key& k) const {
       size_t h = std::hash<int>()(k.chunk) * 0x9e3779b97f4a7c15ull;
-      for (int p : k.pages) h = (h ^ (size_t)(unsigned)p) * 0x100000001b3ull;
+      for (int i = 0; i < k.n; ++i) h = (h ^ (size_t)(unsigned)k.pages[i]) * 0x100000001b3ull;
       return h;
     }
   };
   std::unordered_map<Key, int, KeyHash> index;  // key -> group id
   std::vector<Key> keys;
-  std::vector<std::vector<int>> members;        // rows of each group, in row order
-  std::vector<std::vector<int>> row_chunk_group(rows);
+  std::vector<int> members;                          // rows of each group
+  std::vector<int> row_slot_off(rows + 1), row_slots;  // per row its groups in chunk order, then their slots
+  row_slots.reserve((size_t)rows * 2);
   for (int r = 0; r < rows; ++r) {
     const int npages = pos_of_row[r] / block + 1;
     PGD_CHECK(npages <= max_blocks, kErrShape, "attention plan: position past the block table");
     const int* bt = block_tables + (size_t)seq_of_row[r] * max_blocks;
-    const int nch = (npages + kChunkPages - 1) / kChunkPages;
+    const int nch = (npages + kChunkPages - 1) / kChunkPages, at = (int)row_slots.size();
+    const bool again = r > 0 && seq_of_row[r] == seq_of_row[r - 1];
+    const int whole = again ? std::min(npages, pos_of_row[r - 1] / block + 1) / kChunkPages : 0;
+    row_slot_off[r] = at;
     for (int c = 0; c < nch; ++c) {
-      Key k{c, std::vector<int>(bt + c * kChunkPages, bt + std::min(npages, (c + 1) * kChunkPages))};
-      auto f = index.find(k);
       int gid;
-      if (f == index.end()) {
-        gid = (int)keys.size();
-        index.emplace(k, gid);
-        keys.push_back(std::move(k));
-        members.emplace_back();
+      if (c < whole) {
+        gid = row_slots[row_slot_off[r - 1] + c];
       } else {
-        gid = f->second;
+        const Key k{c, std::min(kChunkPages, npages - c * kChunkPages), bt + c * kChunkPages};
+        const auto f = index.emplace(k, (int)keys.size());
+        gid = f.first->second;
+        if (f.second) {
+          keys.push_back(k);
+          members.push_back(0);
+        }
       }
-      members[gid].push_back(r);
-      row_chunk_group[r].push_back(gid);
+      ++members[gid];
+      row_slots.push_back(gid);
     }
   }
+  row_slot_off[rows] = (int)row_slots.size();
   // items: each group's queries (row-major over its rows, G heads per row) in
   // runs of 16, one matrix-core tile; a query's result does not depend on the
   // other queries of its tile, so tiles may cut between a row's heads
-  std::vector<int> items, pages, item_rows;
-  std::vector<std::vector<int>> group_slot0(keys.size());  // slot of each member
+  std::vector<int> items, pages, item_rows(row_slots.size());
+  std::vector<int> next(keys.size());  // each group's next free slot
+  int base = 0;
   for (size_t gi = 0; gi < keys.size(); ++gi) {
     const int page_off = (int)pages.size();
-    pages.insert(pages.end(), keys[gi].pages.begin(), keys[gi].pages.end());
-    const auto& mem = members[gi];
-    const int base = (int)item_rows.size();
-    for (size_t k = 0; k < mem.size(); ++k) {
-      group_slot0[gi].push_back(base + (int)k);
-      item_rows.push_back(mem[k]);
-    }
-    const int nqs = (int)mem.size() * group;
+    pages.insert(pages.end(), keys[gi].pages, keys[gi].pages + keys[gi].n);
+    const int nqs = members[gi] * group;
     for (int qs = 0; qs < nqs; qs += qpi)
-      items.insert(items.end(), {page_off, (int)keys[gi].pages.size(), base + qs / group, qs % group,
-                                 std::min(qpi, nqs - qs), keys[gi].chunk});
+      items.insert(items.end(), {page_off, keys[gi].n, base + qs / group, qs % group, std::min(qpi, nqs - qs),
+                                 keys[gi].chunk});
+    next[gi] = base;
+    base += members[gi];
   }
-  // row -> slots in chunk order
-  std::vector<int> row_slot_off(rows + 1), row_slots;
-  std::vector<size_t> cursor(keys.size(), 0);
-  for (int r = 0; r < rows; ++r) {
-    row_slot_off[r] = (int)row_slots.size();
-    for (int gid : row_chunk_group[r]) row_slots.push_back(group_slot0[gid][cursor[gid]++]);
-  }
-  row_slot_off[rows] = (int)row_slots.size();
+  for (int r = 0; r < rows; ++r)
+    for (int i = row_slot_off[r]; i < row_slot_off[r + 1]; ++i) {
+      const int slot = next[row_slots[i]]++;
+      item_rows[slot] = r;
+      row_slots[i] = slot;
+    }
   // layout: header {n_items, n_slots, off_items, off_pages, off_item_rows, off_row_slot_off, off_row_slots}
   const int hdr = 8;
   out.assign(hdr, 0);

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <exception>
+#include <mutex>
 #include <new>
 #include <string>
 
@@ -13,6 +14,14 @@
 struct pgd_dev {
   int ordinal;
   hipStream_t stream = nullptr;
+  // pgd_attn_decode_dev's staging, grown on demand and kept: pinned row
+  // metadata and plan, and the plan's device copy. One call at a time (mu);
+  // each call waits for the stream before the host writes any of it.
+  struct AttnStage {
+    std::mutex mu;
+    int *meta = nullptr, *plan = nullptr, *plan_dev = nullptr;
+    size_t meta_ints = 0, plan_ints = 0;
+  } attn;
   explicit pgd_dev(int ord) : ordinal(ord) {
     int prev = 0;
     PGD_HIP(hipGetDevice(&prev));
@@ -28,6 +37,9 @@ struct pgd_dev {
       (void)hipSetDevice(ordinal);
       (void)hipStreamSynchronize(stream);
       (void)hipStreamDestroy(stream);
+      if (attn.meta) (void)hipHostFree(attn.meta);
+      if (attn.plan) (void)hipHostFree(attn.plan);
+      if (attn.plan_dev) (void)hipFree(attn.plan_dev);
       (void)hipSetDevice(prev);
     }
   }

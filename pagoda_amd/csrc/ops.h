@@ -134,6 +134,12 @@ struct AttnPlan {
 void build_attn_plan(const int* seq_of_row, const int* pos_of_row, int rows, const int* block_tables,
                      int max_blocks, int block, int group, int head_dim, std::vector<int>& out);
 AttnPlan attn_plan_view(const int* host, const int* dev);
+// Queues a copy of a launch's row metadata from the device into host memory
+// `out` ([2 + 2 rows + table_cap] ints, device accessible): the number of
+// sequences, the lowest sequence index, seq_of_row, pos_of_row, and the
+// sequences' block tables if they are at most table_cap ints.
+void attn_fetch_meta(const int* seq_of_row, const int* pos_of_row, const int* block_tables, int rows, int max_blocks,
+                     int* out, long long table_cap, hipStream_t s);
 // The same attention in the CPU path's exact operation order (sequential dot,
 // sum and weighted sum; exp correctly rounded): bit-equal to the CPU
 // restatement. out [rows, heads, head_dim]; max_len: the longest context of

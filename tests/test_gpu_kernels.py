@@ -334,3 +334,44 @@ def test_paged_attention_shared_trunk(dev, heads, kvh, hd):
         np.testing.assert_array_equal(run([r])[0].view(np.uint32), out[r].view(np.uint32))
     for p in pools:
         dev.free(p)
+
+
+def test_attention_metadata_staging():
+    """One row whose sequence index lies far past the row count (block tables
+    larger than the staging of a fresh device handle), then many rows (the
+    staging grows), then the one row again: the same bits as sequence 0 of a
+    one-row table; a negative index is refused in between."""
+    from pagoda_amd import Device, PagodaError
+    from pagoda_amd._lib import call
+    import ctypes as C
+
+    dev = Device("hip")
+    rng = np.random.default_rng(9)
+    heads, kvh, hd, nb, nseq, ctx = 4, 2, 64, 64, 41, 200
+    k, v = (rng.normal(0, 1, (nb, kvh, 16, hd)).astype(np.float32) for _ in range(2))
+    table = np.zeros((nseq, nb), np.int32)
+    table[:] = rng.permutation(nb)
+    q = rng.normal(0, 1, (300, heads, hd)).astype(np.float32)
+    dk, dv, dt, dq, out = dev.upload(k), dev.upload(v), dev.upload(table), dev.upload(q), dev.alloc(q.nbytes)
+
+    def run(seq, pos):
+        ds, dp = dev.upload(np.asarray(seq, np.int32)), dev.upload(np.asarray(pos, np.int32))
+        try:
+            call("pgd_attn_decode_dev", dev.handle, heads, kvh, hd, 16, C.c_void_p(dq), None, C.c_void_p(dk),
+                 C.c_void_p(dv), C.c_void_p(ds), C.c_void_p(dp), C.c_void_p(dt), nb, len(seq), C.c_void_p(out))
+            return dev.download(out, (len(seq), heads, hd), np.float32)
+        finally:
+            dev.free(ds)
+            dev.free(dp)
+
+    ref = run([0], [ctx - 1])
+    far = run([nseq - 1], [ctx - 1])
+    with pytest.raises(PagodaError):
+        run([0, -1], [3, 3])
+    many = run([r % nseq for r in range(300)], [ctx - 1] * 300)
+    again = run([nseq - 1], [ctx - 1])
+    for got in (far[0], many[0], again[0]):
+        np.testing.assert_array_equal(got.view(np.uint32), ref[0].view(np.uint32))
+    for p in (dk, dv, dt, dq, out):
+        dev.free(p)
+    dev.close()
