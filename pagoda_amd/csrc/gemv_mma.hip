@@ -1052,13 +1052,14 @@ void launch_pair(const GemvArgs& a, const uint4* XA, const float* CA, int nb, hi
   }
 }
 
-// batches of at least two 128-row blocks take the GEMM (weights read once per
-// 128 rows) when it has work for most of the chip; below that, the GEMV
-// kernels' K splits keep more compute units streaming (measured on MI355X:
-// the qkv projection at 128 rows 183 us as 56 GEMM workgroups against 91 us
-// as two 64-row GEMV launches; 160-row steps of config 5 ran 13% slower
-// through one full and one mostly empty GEMM block)
-constexpr int kGemmRows = 128;
+// Batches of at least 256 rows take the GEMM (weights read once per 64 rows)
+// when it has work for half of the chip; below that, the GEMV kernels' K splits
+// keep more compute units streaming, and steps of up to 255 rows keep one
+// arithmetic per row whatever the batch. All rows go, a partly filled last block
+// included (1266 rows: 50 rows cost 1/20 of the GEMM, about 40 us of gate/up,
+// against 70 us as a GEMV launch), unless the last activation chunk is stored
+// compact (1..4 rows), which takes the GEMV kernels.
+constexpr int kGemmRows = 256;
 constexpr int kGemmMinWorkgroups = 128;
 
 // Rows [0, rows) of a launch through the GEMM, then the prepared-output emits
@@ -1104,10 +1105,8 @@ void launch_prepped(GemvArgs a, const A8Act& act, hipStream_t s) {
   // chunk of a pair holds more than 4 rows (full operand layout)
   const bool pairs = EPI != EPI_SWIGLU && !sk && a.n_out % 4 == 0;
   int c0 = 0;
-  // whole 128-row blocks through the GEMM (a partly filled block costs a
-  // full one), the rest through the GEMV kernels
-  const int gr = rows / kGemmRows * kGemmRows;
-  if (gr >= 2 * kGemmRows && !a.cout && a.row0 == 0 &&
+  const int tail = rows % 32, gr = tail > 4 ? rows : rows - tail;
+  if (gr >= kGemmRows && !a.cout && a.row0 == 0 &&
       a8_gemm_workgroups(a.n_out, gr, EPI) >= kGemmMinWorkgroups) {
     launch_gemm_rows<EPI>(a, XA, act.CA, gr, s);
     c0 = gr / 32;

@@ -443,6 +443,54 @@ def test_a8_prefill_gemm(dev, rows, epi):
 
 
 
+@pytest.mark.parametrize("n_out,rows,epi", [
+    (8200, 256, "store"),    # 3 subtiles per wave; a partial weight block
+    (8200, 293, "res"),      # a last batch block of 37 rows (its second chunk 5 rows)
+    (8200, 515, "store"),    # 3 rows past whole chunks: the GEMV kernels'
+    (8200, 1030, "res"),     # 4 subtiles per wave; 17 batch blocks (groups of 8, 8 and 1)
+    (4100, 261, "swiglu"),   # the pair, a partial weight block and chunk
+    (4100, 1200, "swiglu"),
+])
+def test_a8_prefill_gemm_tiles(dev, n_out, rows, epi):
+    """The A8 GEMM at the edges of its tiles (launches of enough workgroups to
+    take it; two groups, so both stages and the fold across groups count):
+    against fp64 on the same dequantized weights, and a row's bits the same
+    whichever launch holds it."""
+    from pagoda_amd import Matrix
+    from pagoda_amd.matrix import act_bytes, act_prep_dev
+
+    K = 128
+    m = Matrix.synth(dev, 0, n_out, K, 71, 3, 0.02)
+    u = Matrix.synth(dev, 0, n_out, K, 72, 4, 0.02) if epi == "swiglu" else None
+    rng = np.random.default_rng(rows)
+    x = rng.normal(0, 1, (rows, K)).astype(np.float32)
+    res = rng.normal(0, 1, (rows, n_out)).astype(np.float32)
+
+    def run(r):
+        xd, act, yd = dev.upload(x[:r]), dev.alloc(act_bytes(r, K)), dev.upload(res[:r])
+        act_prep_dev(dev, xd, K, r, K, act)
+        if epi == "swiglu":
+            Matrix.gemv_swiglu_act_dev(m, u, act, r, yd, n_out)
+        else:
+            m.gemv_act_dev(act, r, yd, n_out, yd if epi == "res" else 0, n_out)
+        got = dev.download(yd, (r, n_out), np.float32)
+        for p in (xd, act, yd):
+            dev.free(p)
+        return got
+
+    x64, w64 = x.astype(np.float64), m.dequant().astype(np.float64)
+    if epi == "swiglu":
+        g = x64 @ w64.T
+        ref = g / (1.0 + np.exp(-g)) * (x64 @ u.dequant().astype(np.float64).T)
+    else:
+        ref = x64 @ w64.T + (res if epi == "res" else 0)
+    got = run(rows)
+    assert rel_err(got, ref) < GEMV_TOL, rel_err(got, ref)
+    if rows > 512:
+        np.testing.assert_array_equal(run(512).view(np.uint32), got[:512].view(np.uint32))
+    m.free()
+
+
 @pytest.mark.parametrize("n_out,n_in,rows,dual", [(17408, 5120, 32, True), (17408, 5120, 64, True),
                                                    (17408, 5120, 9, True), (151936, 5120, 32, False)])
 def test_a8_stream_k_repeatable(dev, n_out, n_in, rows, dual):
