@@ -50,7 +50,7 @@ struct GemvArgs {
   // deferred RMSNorm of the input (null: none): rss rows of this launch,
   // rss_nh partials per row, row width rss_n, eps; outputs are scaled by
   // rss_inv() of their row. inv: optional per-launch-row copy of those
-  // factors written by the stream-K kernel for its fix-up kernel.
+  // factors, written by the stream-K kernel for its fix-up kernel or before a GEMM.
   const float* rss;
   int rss_nh, rss_n;
   float rss_eps;
@@ -479,7 +479,7 @@ void run_a8_mma(const GemvArgs& a, const A8Act& act, int epi, hipStream_t s);
 // A8 GEMM for prefill-sized batches: rows [0, rows) of a prepared activation
 // (whose chunks there are in the full, not compact, layout), epilogue STORE,
 // RES or SWIGLU into a.y (no prepared-output emits, no conv)
-void run_a8_gemm(const GemvArgs& a, const uint4* XA, const float* CA, int rows, int epi, hipStream_t s);
+void run_a8_gemm(GemvArgs a, const uint4* XA, const float* CA, int rows, int epi, hipStream_t s);
 // workgroups of that GEMM (256 weight rows, or 128 SwiGLU pairs, by 128 batch rows each)
 int a8_gemm_workgroups(int n_out, int rows, int epi);
 // Stream-K A8 kernel: whether a matrix takes it for 5..32-row launches, and
