@@ -57,7 +57,10 @@ struct GemvArgs {
   float* inv;
   // residual launches only: also emit the next RMSNorm's deferred input from
   // the new rows h = res + W x (operands of h * nw into nact, per-32-column
-  // sums of h^2 into nrss [rows][n_out / 32]); nact.XA null: no
+  // sums of h^2 into nrss [rows][n_out / 32]); nact.XA null: no. In
+  // quantized-activation launches of a few rows nw (null: none) norms the
+  // input instead: x / rms(x) * nw, candle's rms_norm with its order of
+  // additions, eps in rss_eps
   a8act::Dst nact;
   const float* nw;
   float* nrss;
@@ -71,10 +74,6 @@ struct GemvArgs {
   size_t coff;
   float* cout;
   int ldc, conv_n, conv_k;
-  // quantized-activation launches of a few rows (null: none): the input is
-  // x / rms(x) * norm_w, candle's rms_norm with its order of additions
-  const float* norm_w;
-  float norm_eps;
 };
 
 // the causal conv step of one channel for one row: conv_step_kernel's
@@ -469,7 +468,7 @@ void run_q8_gemm_pair(int fmt_a, GemvArgs a, int fmt_b, GemvArgs b, int nrows, h
 bool q8act_pair_ok(int fmt_a, int fmt_b);
 void run_q8act_pair(int fmt_a, const GemvArgs& a, int fmt_b, const GemvArgs& b, int nrows, hipStream_t s);
 // whether launches of nrows rows over tiles16 16-row tiles (nm matrices) can
-// run the input's RMSNorm themselves (GemvArgs.norm_w), and whether that pays:
+// run the input's RMSNorm themselves (GemvArgs.nw), and whether that pays:
 // every workgroup repeats the chain of n_in additions, so only while all of
 // them are resident at once
 bool q8k_norm_ok(int tiles16, int nsb, int n_in, int nrows, int nm);

@@ -350,7 +350,7 @@ __device__ void run_tiles(const GemvArgs& a, int first, int ntiles, int stride, 
   // a wave without a block of its own loads (and drops) the last one
   Raw<FMT> cur, nxt;
   load(cur, first, min(wv, units - 1));
-  quantize<FMT, NORM>(reinterpret_cast<const float*>(a.x), a.ldx, rows, a.n_in, a.norm_w, a.norm_eps, L);
+  quantize<FMT, NORM>(reinterpret_cast<const float*>(a.x), a.ldx, rows, a.n_in, a.nw, a.rss_eps, L);
   __syncthreads();
   for (int tile = first; tile < ntiles; tile += stride) {
     for (int unit = wv; unit < units; unit += nw) {
@@ -493,7 +493,7 @@ void launch_pair(GemvArgs a, GemvArgs b, int nrows, hipStream_t s) {
 template <int FMT>
 void run_epi(const GemvArgs& a, int nrows, int epi, hipStream_t s) {
   if (epi == EPI_SWIGLU) {
-    if (a.norm_w) launch<FMT, EPI_SWIGLU, true>(a, nrows, s);
+    if (a.nw) launch<FMT, EPI_SWIGLU, true>(a, nrows, s);
     else launch<FMT, EPI_SWIGLU, false>(a, nrows, s);
   } else if (epi == EPI_RES) {
     launch<FMT, EPI_RES, false>(a, nrows, s);
@@ -504,7 +504,7 @@ void run_epi(const GemvArgs& a, int nrows, int epi, hipStream_t s) {
 
 template <int FMT, int FMT2>
 void run_pair(const GemvArgs& a, const GemvArgs& b, int nrows, hipStream_t s) {
-  if (a.norm_w) launch_pair<FMT, FMT2, true>(a, b, nrows, s);
+  if (a.nw) launch_pair<FMT, FMT2, true>(a, b, nrows, s);
   else launch_pair<FMT, FMT2, false>(a, b, nrows, s);
 }
 

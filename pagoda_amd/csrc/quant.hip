@@ -696,8 +696,8 @@ void q8act_pair(const QMat& a, float* ya, const QMat& b, float* yb, const float*
   ga.y = ya;
   gb.y = yb;
   ga.ldy = gb.ldy = ldy;
-  ga.norm_w = gb.norm_w = nw;
-  ga.norm_eps = gb.norm_eps = eps;
+  ga.nw = gb.nw = nw;
+  ga.rss_eps = gb.rss_eps = eps;
   run_q8act_pair(a.fmt, ga, b.fmt, gb, nrows, s);
 }
 
@@ -716,8 +716,8 @@ void q8act_swiglu(const QMat& gate, const QMat& up, const float* x, int ldx, con
   a.ldx = ldx;
   a.y = mid;
   a.ldy = ldm;
-  a.norm_w = nw;
-  a.norm_eps = eps;
+  a.nw = nw;
+  a.rss_eps = eps;
   run_q8act(gate.fmt, a, nrows, EPI_SWIGLU, s);
 }
 }  // namespace
