@@ -123,8 +123,6 @@ void qmat_gemv(const QMat& m, const void* x, int x_f16, int ldx, int nrows, floa
 // output is an integer block dot scaled in f32.
 void qmat_gemv_q8act(const QMat& m, const float* x, int ldx, int nrows, float* y, int ldy, const float* res, int ldres,
                      hipStream_t s);
-void qmat_gemv_swiglu_q8act(const QMat& gate, const QMat& up, const float* x, int ldx, int nrows, float* mid, int ldm,
-                            hipStream_t s);
 // qmat_gemv_q8act of two matrices over the same input rows in one launch
 // (ya = A.x, yb = B.x, both with row stride ldy), bit-equal to two calls;
 // qmat_q8act_pairable says whether two matrices can share a launch.
@@ -132,9 +130,10 @@ bool qmat_q8act_pairable(const QMat& a, const QMat& b);
 void qmat_gemv_q8act_pair(const QMat& a, float* ya, const QMat& b, float* yb, const float* x, int ldx, int nrows,
                           int ldy, hipStream_t s);
 
-// The two calls above over rows normed first (rmsnorm_rows mode 2: x / rms * nw,
-// the squares summed left to right): inside the launch where that pays, else
-// through xn (at least nrows rows of stride ldx); the same bits either way.
+// The pair, and silu(gate.x) * (up.x) in the same arithmetic, over rows normed
+// first (rmsnorm_rows mode 2: x / rms * nw, the squares summed left to right):
+// inside the launch where that pays, else through xn (at least nrows rows of
+// stride ldx); the same bits either way.
 void qmat_gemv_swiglu_q8act_norm(const QMat& gate, const QMat& up, const float* x, int ldx, const float* nw, float eps,
                                  float* xn, int nrows, float* mid, int ldm, hipStream_t s);
 void qmat_gemv_q8act_pair_norm(const QMat& a, float* ya, const QMat& b, float* yb, const float* x, int ldx,

@@ -735,11 +735,6 @@ void qmat_gemv_q8act_pair_norm(const QMat& a, float* ya, const QMat& b, float* y
   q8act_pair(a, ya, b, yb, xn, ldx, nullptr, 0.0f, nrows, ldy, s);
 }
 
-void qmat_gemv_swiglu_q8act(const QMat& gate, const QMat& up, const float* x, int ldx, int nrows, float* mid, int ldm,
-                            hipStream_t s) {
-  q8act_swiglu(gate, up, x, ldx, nullptr, 0.0f, nrows, mid, ldm, s);
-}
-
 void qmat_gemv_swiglu_q8act_norm(const QMat& gate, const QMat& up, const float* x, int ldx, const float* nw, float eps,
                                  float* xn, int nrows, float* mid, int ldm, hipStream_t s) {
   if (gemv::q8act_norm_fused(gate.fmt, tiles16(gate), gate.nsb, gate.n_in, nrows, 2))
