@@ -27,6 +27,8 @@
 // block). Measured against 16 rows per launch on the vector ALUs: 4864 x 896
 // Q4_K 81 rows 138 -> 11.5 us, 333 rows 547 -> 22.5 us, 1000 rows 1643 ->
 // 47 us; 896 x 4864 Q6_K 81 rows 632 -> 27 us, 1000 rows 7786 -> 54 us.
+#include <mutex>
+
 #include "common.h"
 #include "gemv_impl.h"
 #include "quant.h"
@@ -514,11 +516,17 @@ void advance(GemvArgs& a, int rows) {
   if (a.res) a.res += (size_t)rows * a.ldres;
 }
 
+// The operands lie in the stream's scratch between the two launches. Held over
+// both, so that no other host thread's call on the stream is queued between
+// them or replaces the buffer.
+std::mutex g_operands;
+
 }  // namespace
 
 void run_q8_gemm(int fmt, GemvArgs a, int nrows, int epi, hipStream_t s) {
   for (int r0 = 0; r0 < nrows; r0 += kRowChunk) {
     const int rows = min(kRowChunk, nrows - r0);
+    std::lock_guard<std::mutex> lock(g_operands);
     const char* act = prep(reinterpret_cast<const float*>(a.x), a.ldx, rows, a.n_in, a.nsb, s);
     if (fmt == FMT_Q4K) run_epi<FMT_Q4K>(a, act, rows, epi, s);
     else run_epi<FMT_Q6K>(a, act, rows, epi, s);
@@ -529,6 +537,7 @@ void run_q8_gemm(int fmt, GemvArgs a, int nrows, int epi, hipStream_t s) {
 void run_q8_gemm_pair(int fmt_a, GemvArgs a, int fmt_b, GemvArgs b, int nrows, hipStream_t s) {
   for (int r0 = 0; r0 < nrows; r0 += kRowChunk) {
     const int rows = min(kRowChunk, nrows - r0);
+    std::lock_guard<std::mutex> lock(g_operands);
     const char* act = prep(reinterpret_cast<const float*>(a.x), a.ldx, rows, a.n_in, a.nsb, s);
     if (fmt_a == FMT_Q4K && fmt_b == FMT_Q4K) run_pair<FMT_Q4K, FMT_Q4K>(a, b, act, rows, s);
     else if (fmt_a == FMT_Q4K) run_pair<FMT_Q4K, FMT_Q6K>(a, b, act, rows, s);

@@ -216,3 +216,53 @@ def test_q8act_kernels_match_oracle(dev, fmt, n_out, n_in, rows):
     for p in (xd, yd, y2, rd):
         dev.free(p)
     m.free()
+
+
+@pytest.mark.parametrize("pair", [False, True])
+def test_q8act_calls_from_two_threads(dev, pair):
+    """Two host threads issue matrix-core launches on one device handle without
+    a lock of their own: each call's product takes its own rows' operands,
+    whatever the other thread queues meanwhile (other rows, widths and buffer
+    sizes). Every output is bit-equal to the same call on one thread."""
+    import threading
+
+    from pagoda_amd import Matrix
+
+    calls, jobs, bad = 150, [], []
+    for fmt, n_out, n_in, rows, seed in ((1, 48, 1024, 33, 1), (2, 80, 512, 70, 2)):
+        m, _ = make(dev, fmt, n_out, n_in, seed)
+        x = np.random.default_rng(seed).normal(0, 1, (rows, n_in)).astype(np.float32)
+        out = dev.upload(np.zeros((calls + 1, rows, 2, n_out), np.float32))
+        jobs.append((m, dev.upload(x), n_in, rows, n_out, out))
+
+    def issue(job, i):
+        m, xd, n_in, rows, n_out, out = job
+        y = out + i * rows * 2 * n_out * 4
+        if pair:
+            m.gemv_q8act_pair_dev(y, m, y + n_out * 4, xd, n_in, rows, 2 * n_out)
+        else:
+            m.gemv_q8act_dev(xd, n_in, rows, y, 2 * n_out)
+
+    def work(job):
+        try:
+            for i in range(1, calls + 1):
+                issue(job, i)
+        except Exception as e:  # reported by the main thread
+            bad.append(e)
+
+    for job in jobs:
+        issue(job, 0)
+        dev.sync()
+    threads = [threading.Thread(target=work, args=(job,)) for job in jobs]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad, bad
+    for m, xd, n_in, rows, n_out, out in jobs:
+        got = dev.download(out, (calls + 1, rows, 2, n_out), np.float32).view(np.uint32)
+        wrong = [i for i in range(1, calls + 1) if not np.array_equal(got[i], got[0])]
+        assert not wrong, wrong
+        dev.free(xd)
+        dev.free(out)
+        m.free()
