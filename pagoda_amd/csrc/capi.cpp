@@ -348,6 +348,20 @@ int pgd_gdn_prefill_dev(pgd_dev* dev, int k_heads, int v_heads, const float* con
                   rows, max_rows, out);
 }
 
+namespace {
+// ints from p to the end of its device allocation; false if the runtime knows none
+bool ints_at(const int* p, size_t& n) {
+  hipDeviceptr_t base = nullptr;
+  size_t bytes = 0;
+  if (hipMemGetAddressRange(&base, &bytes, const_cast<int*>(p)) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  n = (bytes - (reinterpret_cast<uintptr_t>(p) - reinterpret_cast<uintptr_t>(base))) / sizeof(int);
+  return true;
+}
+}  // namespace
+
 int pgd_attn_decode_dev(pgd_dev* dev, int heads, int kv_heads, int head_dim, int block, const float* q,
                         const float* gate, const float* k_pool, const float* v_pool, const int* seq_of_row,
                         const int* pos_of_row, const int* block_tables, int max_blocks, int rows, float* out) {
@@ -361,10 +375,13 @@ int pgd_attn_decode_dev(pgd_dev* dev, int heads, int kv_heads, int head_dim, int
     if (rows == 0) return;
     PGD_CHECK(kv_heads > 0 && heads % kv_heads == 0, kErrShape, "heads must be a multiple of kv_heads");
     // The plan is built from the row metadata on the host: one small kernel
-    // writes it to pinned memory (three copies of their own before, and an
-    // allocation, a free and a second wait around the launch: 167 -> 93 us for
-    // 32 rows whose kernels take 60), the call waits for that, and the launch
-    // itself is only queued.
+    // writes it to pinned memory, the call waits for that, and the launch itself
+    // is only queued. The kernel reads no further than the arrays' allocations:
+    // shorter ones are an error, as they are to a copy.
+    size_t n_seq = 0, n_pos = 0, n_bt = 0;
+    const bool bt_known = ints_at(block_tables, n_bt);
+    PGD_CHECK((!ints_at(seq_of_row, n_seq) || n_seq >= (size_t)rows) && (!ints_at(pos_of_row, n_pos) || n_pos >= (size_t)rows),
+              kErrHip, "row metadata shorter than the rows");
     std::lock_guard<std::mutex> lock(dev->attn.mu);
     pgd_dev::AttnStage& g = dev->attn;
     // room for the tables of as many sequences as rows, up to 4 MiB
@@ -379,7 +396,8 @@ int pgd_attn_decode_dev(pgd_dev* dev, int heads, int kv_heads, int head_dim, int
     };
     if (g.meta_ints < want) PGD_HIP(hipStreamSynchronize(dev->stream));
     pinned(g.meta, g.meta_ints, want);
-    const size_t fixed = 2 + 2 * (size_t)rows, cap = g.meta_ints - fixed;
+    // (tables outside any known allocation take the copy below)
+    const size_t fixed = 2 + 2 * (size_t)rows, cap = std::min(g.meta_ints - fixed, n_bt);
     attn_fetch_meta(seq_of_row, pos_of_row, block_tables, rows, max_blocks, g.meta, (long long)cap, dev->stream);
     PGD_HIP(hipStreamSynchronize(dev->stream));
     PGD_CHECK(g.meta[1] >= 0, kErrArg, "negative sequence index");
@@ -387,6 +405,7 @@ int pgd_attn_decode_dev(pgd_dev* dev, int heads, int kv_heads, int head_dim, int
     const size_t tables = (size_t)(unsigned)g.meta[0] * max_blocks;
     std::vector<int> far;
     if (tables > cap) {
+      PGD_CHECK(!bt_known || tables <= n_bt, kErrHip, "sequence index past the block tables");
       far.resize(tables);
       PGD_HIP(hipMemcpy(far.data(), block_tables, tables * sizeof(int), hipMemcpyDeviceToHost));
       h_bt = far.data();

@@ -340,7 +340,9 @@ def test_attention_metadata_staging():
     """One row whose sequence index lies far past the row count (block tables
     larger than the staging of a fresh device handle), then many rows (the
     staging grows), then the one row again: the same bits as sequence 0 of a
-    one-row table; a negative index is refused in between."""
+    one-row table; a negative index is refused in between, and with the staging
+    grown so are an index past the end of the block tables' allocation (its
+    table would fit the staging) and row arrays shorter than the rows."""
     from pagoda_amd import Device, PagodaError
     from pagoda_amd._lib import call
     import ctypes as C
@@ -369,6 +371,16 @@ def test_attention_metadata_staging():
     with pytest.raises(PagodaError):
         run([0, -1], [3, 3])
     many = run([r % nseq for r in range(300)], [ctx - 1] * 300)
+    for idx in (nseq + 10, 500):
+        with pytest.raises(PagodaError):
+            run([0, idx], [3, 3])
+    short, whole = dev.upload(np.zeros(8, np.int32)), dev.upload(np.zeros(300, np.int32))
+    for seq, pos in ((short, whole), (whole, short)):
+        with pytest.raises(PagodaError):
+            call("pgd_attn_decode_dev", dev.handle, heads, kvh, hd, 16, C.c_void_p(dq), None, C.c_void_p(dk),
+                 C.c_void_p(dv), C.c_void_p(seq), C.c_void_p(pos), C.c_void_p(dt), nb, 300, C.c_void_p(out))
+    dev.free(short)
+    dev.free(whole)
     again = run([nseq - 1], [ctx - 1])
     for got in (far[0], many[0], again[0]):
         np.testing.assert_array_equal(got.view(np.uint32), ref[0].view(np.uint32))
