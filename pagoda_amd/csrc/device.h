@@ -10,6 +10,7 @@
 #include <string>
 
 #include "common.h"
+#include "quant.h"
 
 struct pgd_dev {
   int ordinal;
@@ -36,6 +37,7 @@ struct pgd_dev {
       (void)hipGetDevice(&prev);
       (void)hipSetDevice(ordinal);
       (void)hipStreamSynchronize(stream);
+      pgd::gemv::scratch_release(stream);
       (void)hipStreamDestroy(stream);
       if (attn.meta) (void)hipHostFree(attn.meta);
       if (attn.plan) (void)hipHostFree(attn.plan);

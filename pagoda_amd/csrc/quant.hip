@@ -431,6 +431,32 @@ std::atomic<uint64_t> g_scratch_epoch{0};
 
 uint64_t scratch_epoch() { return g_scratch_epoch.load(std::memory_order_relaxed); }
 
+namespace {
+struct Scratch {
+  std::mutex mu;
+  std::map<std::pair<hipStream_t, int>, std::pair<void*, size_t>> bufs;
+};
+// (never destroyed: a device handle may be closed during exit)
+Scratch& scratch() {
+  static Scratch* all = new Scratch;
+  return *all;
+}
+}  // namespace
+
+void scratch_release(hipStream_t s) {
+  Scratch& all = scratch();
+  std::lock_guard<std::mutex> lock(all.mu);
+  for (auto it = all.bufs.begin(); it != all.bufs.end();) {
+    if (it->first.first != s) {
+      ++it;
+      continue;
+    }
+    if (it->second.first) (void)hipFree(it->second.first);
+    g_scratch_epoch.fetch_add(1, std::memory_order_relaxed);
+    it = all.bufs.erase(it);
+  }
+}
+
 void* gemv_scratch(hipStream_t s, size_t bytes, int slot) {
   if (ScratchArena* ar = t_arena) {
     PGD_CHECK(slot >= 0 && slot < 8, kErrArg, "scratch slot");
@@ -444,10 +470,9 @@ void* gemv_scratch(hipStream_t s, size_t bytes, int slot) {
     }
     return ar->base + ar->off[slot];
   }
-  static std::mutex mu;
-  static std::map<std::pair<hipStream_t, int>, std::pair<void*, size_t>> bufs;
-  std::lock_guard<std::mutex> lock(mu);
-  auto& e = bufs[{s, slot}];
+  Scratch& all = scratch();
+  std::lock_guard<std::mutex> lock(all.mu);
+  auto& e = all.bufs[{s, slot}];
   if (e.second < bytes) {
     if (e.first) {
       PGD_HIP(hipStreamSynchronize(s));

@@ -266,3 +266,38 @@ def test_q8act_calls_from_two_threads(dev, pair):
         dev.free(xd)
         dev.free(out)
         m.free()
+
+
+def test_device_close_gives_scratch_back():
+    """Launch scratch is kept per device handle (here the prepared operands of
+    1024 rows of 4096, 9 MB a handle) and freed with it."""
+    import ctypes as C
+
+    from pagoda_amd import Device, Matrix
+
+    def used():
+        free, total = C.c_size_t(), C.c_size_t()
+        # the runtime library the backend has loaded
+        assert C.CDLL("libamdhip64.so.7").hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return total.value - free.value
+
+    def run(n):
+        devs = [Device("hip") for _ in range(n)]
+        for d in devs:
+            m = Matrix.synth(d, 1, 16, 4096, 1, 1)
+            xd, yd = d.alloc(1024 * 4096 * 4), d.alloc(1024 * 16 * 4)
+            m.gemv_q8act_dev(xd, 4096, 1024, yd, 16)
+            d.sync()
+            m.free()
+            d.free(xd)
+            d.free(yd)
+        held = used()
+        for d in devs:
+            d.close()
+        return held
+
+    run(1)
+    before = used()
+    held = run(6)
+    assert held - before > 48 << 20, (held, before)
+    assert used() - before < 16 << 20, (used(), before)
