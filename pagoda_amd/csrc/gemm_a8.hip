@@ -350,6 +350,19 @@ int a8_gemm_workgroups(int n_out, int rows, int epi) {
   return wblocks(n_out, pick_ns(n_out, rows, epi), epi) * cblocks(rows);
 }
 
+// Microseconds of the GEMM, to compare with the GEMV kernels: a round of 512
+// workgroups takes 33 ns per weight column with four subtiles per wave and 28
+// with three, one of at most 256 half of that (0.42 behind whole rounds), in
+// between linear. Measured within 10% for 4096..17408 columns and 256..2048
+// rows of 2048..17408 outputs and SwiGLU pairs.
+double a8_gemm_us(int n_out, int n_in, int rows, int epi) {
+  const int ns = pick_ns(n_out, rows, epi), wg = wblocks(n_out, ns, epi) * cblocks(rows);
+  const int whole = wg / 512, rest = wg % 512;
+  const double round = ns == 4 ? 1.0 : 0.85;
+  const double part = rest == 0 ? 0.0 : rest > 256 ? (0.57 + 0.43 * (rest - 256) / 256) * round : whole ? 0.42 : 0.5;
+  return 5.0 + 0.0332 * n_in * (whole * round + part);
+}
+
 void run_a8_gemm(GemvArgs a, const uint4* XA, const float* CA, int rows, int epi, hipStream_t s) {
   PGD_CHECK(rows > 0 && (rows % 32 == 0 || rows % 32 > 4), kErrShape,
             "the A8 GEMM takes activation chunks in the full (not compact) layout");

@@ -479,8 +479,10 @@ void run_a8_mma(const GemvArgs& a, const A8Act& act, int epi, hipStream_t s);
 // (whose chunks there are in the full, not compact, layout), epilogue STORE,
 // RES or SWIGLU into a.y (no prepared-output emits, no conv)
 void run_a8_gemm(GemvArgs a, const uint4* XA, const float* CA, int rows, int epi, hipStream_t s);
-// workgroups of that GEMM (256 weight rows, or 128 SwiGLU pairs, by 128 batch rows each)
+// workgroups of that GEMM (256 or 192 weight rows, or 128 SwiGLU pairs, by 64
+// batch rows each) and its estimated microseconds
 int a8_gemm_workgroups(int n_out, int rows, int epi);
+double a8_gemm_us(int n_out, int n_in, int rows, int epi);
 // Stream-K A8 kernel: whether a matrix takes it for 5..32-row launches, and
 // one launch of 5..32 rows (operand chunk XA / CA of the prepared activations)
 bool a8_sk_wanted(const GemvArgs& a, int epi);

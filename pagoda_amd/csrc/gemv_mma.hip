@@ -1052,15 +1052,46 @@ void launch_pair(const GemvArgs& a, const uint4* XA, const float* CA, int nb, hi
   }
 }
 
-// Batches of at least 256 rows take the GEMM (weights read once per 64 rows)
-// when it has work for half of the chip; below that, the GEMV kernels' K splits
-// keep more compute units streaming, and steps of up to 255 rows keep one
-// arithmetic per row whatever the batch. All rows go, a partly filled last block
-// included (1266 rows: 50 rows cost 1/20 of the GEMM, about 40 us of gate/up,
-// against 70 us as a GEMV launch), unless the last activation chunk is stored
-// compact (1..4 rows), which takes the GEMV kernels.
+// Batches of at least 256 rows may take the GEMM (weights read once per 64
+// rows), when it has at least 128 workgroups; steps of up to 255 rows keep one
+// arithmetic per row whatever the batch. gemm_rows() says how many of a
+// launch's rows it takes.
 constexpr int kGemmRows = 256;
 constexpr int kGemmMinWorkgroups = 128;
+
+// Microseconds of the GEMV kernels: launches of 64 rows (plain matrices, a
+// last one of up to 32 rows about half) or of 32 (SwiGLU). Measured for 64
+// rows of 5120 x 17408 47 us, 5120 x 6144 23, 5120 x 4096 18, 12352 x 5120 38,
+// for 32 of the 17408 x 5120 pair 38 and the 9728 x 2560 pair 20.
+double gemv_us(int n_out, int n_in, int rows, int epi) {
+  const double weights = (double)n_out * n_in * 1e-6;
+  if (epi == EPI_SWIGLU) return (13.5 + 0.274 * weights) * ((rows + 31) / 32);
+  const int rest = rows % 64;
+  return (7.0 + 0.46 * weights) * (rows / 64 + (rest == 0 ? 0.0 : rest <= 32 ? 0.55 : 1.0));
+}
+
+// Rows [0, r) of a launch for the GEMM, the rest for the GEMV kernels: none,
+// all, or all but the last one or two batch blocks, whichever is estimated
+// fastest (less than all: by 5%). A GEMM round takes its time however few of
+// its workgroups there are, so a few rows of a long K are the GEMV kernels'
+// (5120 x 17408 at 261 rows 290 us as 135 workgroups, 214 as GEMV launches; at
+// 390 rows 291 against 310), and so are rows that would start another round
+// (8192 x 5120 at 1061 rows 207 us, 195 with the last 37 rows apart). A last
+// activation chunk of 1..4 rows is stored compact, which the GEMV kernels take.
+int gemm_rows(int n_out, int n_in, int rows, int epi) {
+  const int tail = rows % 32, all = tail > 4 ? rows : rows - tail;
+  int take = 0;
+  double best = gemv_us(n_out, n_in, rows, epi);
+  for (int less = 0; less <= 2; ++less) {
+    const int r = less ? ((all + 63) / 64 - less) * 64 : all;
+    if (r < kGemmRows || a8_gemm_workgroups(n_out, r, epi) < kGemmMinWorkgroups) break;
+    const double us = (a8_gemm_us(n_out, n_in, r, epi) + gemv_us(n_out, n_in, rows - r, epi)) * (less ? 1.05 : 1.0);
+    if (us >= best) continue;
+    best = us;
+    take = r;
+  }
+  return take;
+}
 
 // Rows [0, rows) of a launch through the GEMM, then the prepared-output emits
 // the GEMV epilogues would have fused (the next RMSNorm's deferred input, the
@@ -1105,9 +1136,8 @@ void launch_prepped(GemvArgs a, const A8Act& act, hipStream_t s) {
   // chunk of a pair holds more than 4 rows (full operand layout)
   const bool pairs = EPI != EPI_SWIGLU && !sk && a.n_out % 4 == 0;
   int c0 = 0;
-  const int tail = rows % 32, gr = tail > 4 ? rows : rows - tail;
-  if (gr >= kGemmRows && !a.cout && a.row0 == 0 &&
-      a8_gemm_workgroups(a.n_out, gr, EPI) >= kGemmMinWorkgroups) {
+  const int gr = !a.cout && a.row0 == 0 ? gemm_rows(a.n_out, a.n_in, rows, EPI) : 0;
+  if (gr > 0) {
     launch_gemm_rows<EPI>(a, XA, act.CA, gr, s);
     c0 = gr / 32;
     rows -= gr;

@@ -491,6 +491,60 @@ def test_a8_prefill_gemm_tiles(dev, n_out, rows, epi):
     m.free()
 
 
+@pytest.mark.parametrize("n_out,n_in,epi,rows,gemm", [
+    (5120, 17408, "res", 261, 0),        # 135 GEMM workgroups of a long K: the GEMV kernels are faster
+    (5120, 17408, "res", 384, 0),
+    (5120, 17408, "res", 448, 448),      # from about 390 rows on the GEMM is
+    (8192, 5120, "store", 1061, 1024),   # the last 37 rows would start another round of workgroups
+    (9728, 2560, "swiglu", 390, 384),
+    (9728, 2560, "swiglu", 387, 384),    # 3 rows past whole chunks (stored compact)
+])
+def test_a8_gemm_takes_the_rows_it_is_faster_for(dev, n_out, n_in, epi, rows, gemm):
+    """Which rows of a batch the A8 GEMM computes (rows below `gemm`), told from
+    the others by their bits: those of a 512-row launch. The GEMV kernels give a
+    row the bits it has in a 64-row launch, or (1 to 4 rows left over, another
+    kernel) in a launch of the left-over rows. Some rows against fp64."""
+    from pagoda_amd import Matrix
+    from pagoda_amd.matrix import act_bytes, act_prep_dev
+
+    m = Matrix.synth(dev, 0, n_out, n_in, 81, 3, 0.02)
+    u = Matrix.synth(dev, 0, n_out, n_in, 82, 4, 0.02) if epi == "swiglu" else None
+    rng = np.random.default_rng(rows)
+    x = rng.normal(0, 1, (rows, n_in)).astype(np.float32)
+    res = rng.normal(0, 1, (rows, n_out)).astype(np.float32)
+
+    def run(at):
+        r = len(at)
+        xd, act, yd = dev.upload(x[at]), dev.alloc(act_bytes(r, n_in)), dev.upload(res[at])
+        act_prep_dev(dev, xd, n_in, r, n_in, act)
+        if u:
+            Matrix.gemv_swiglu_act_dev(m, u, act, r, yd, n_out)
+        else:
+            m.gemv_act_dev(act, r, yd, n_out, yd if epi == "res" else 0, n_out)
+        got = dev.download(yd, (r, n_out), np.float32)
+        for p in (xd, act, yd):
+            dev.free(p)
+        return got
+
+    got = run(np.arange(rows))
+    few = np.unique([0, 63, 64, rows // 2, max(gemm - 1, 0), min(gemm, rows - 1), rows - 1])
+    gemv, mm = run(np.resize(few, 64)), run(np.resize(few, 512))
+    left = run(np.arange(gemm, rows)) if rows - gemm in range(1, 64) else None
+    for i, r in enumerate(few):
+        assert not np.array_equal(gemv[i], mm[i])
+        want = mm[i] if r < gemm else gemv[i] if left is None else left[r - gemm]
+        np.testing.assert_array_equal(got[r].view(np.uint32), want.view(np.uint32), err_msg=f"row {r}")
+    x64, w64 = x[few].astype(np.float64), m.dequant().astype(np.float64)
+    ref = x64 @ w64.T
+    if u:
+        ref = ref / (1.0 + np.exp(-ref)) * (x64 @ u.dequant().astype(np.float64).T)
+        u.free()
+    elif epi == "res":
+        ref += res[few]
+    assert rel_err(got[few], ref) < GEMV_TOL, rel_err(got[few], ref)
+    m.free()
+
+
 @pytest.mark.parametrize("n_out,n_in,rows,dual", [(17408, 5120, 32, True), (17408, 5120, 64, True),
                                                    (17408, 5120, 9, True), (151936, 5120, 32, False)])
 def test_a8_stream_k_repeatable(dev, n_out, n_in, rows, dual):
