@@ -468,9 +468,8 @@ void run_q8_gemm_pair(int fmt_a, GemvArgs a, int fmt_b, GemvArgs b, int nrows, h
 bool q8act_pair_ok(int fmt_a, int fmt_b);
 void run_q8act_pair(int fmt_a, const GemvArgs& a, int fmt_b, const GemvArgs& b, int nrows, hipStream_t s);
 // whether launches of nrows rows over tiles16 16-row tiles (nm matrices) can
-// run the input's RMSNorm themselves (GemvArgs.nw), and whether that pays:
-// every workgroup repeats the chain of n_in additions, so only while all of
-// them are resident at once
+// run the input's RMSNorm themselves (GemvArgs.nw) with every workgroup
+// resident at once, and whether they take that form
 bool q8k_norm_ok(int tiles16, int nsb, int n_in, int nrows, int nm);
 bool q8act_norm_fused(int fmt, int tiles16, int nsb, int n_in, int nrows, int nm);
 // A8 on the matrix cores (f32 activations)

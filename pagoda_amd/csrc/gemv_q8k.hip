@@ -522,9 +522,19 @@ void run_q8k_gemv_pair(int fmt_a, const GemvArgs& a, int fmt_b, const GemvArgs& 
   else run_pair<FMT_Q6K, FMT_Q6K>(a, b, nrows, s);
 }
 
+// Every workgroup of a launch with the norm repeats the chain of n_in additions,
+// so the norm goes in only where all of them are resident at once: per CU the
+// LDS, and 16 waves (the kernels' 128 registers), at most two. A second round
+// repeats the chain. us per layer of a decode step, norm inside / in its own
+// launch: 4608 x 3584 (288 workgroups of 14 waves) 1 row 139.5 / 134.1, 5 rows
+// 142 / 133; gate/up 8192 x 2048 (512 of 16 waves) 76.1 / 71.2; in one round
+// (1152 x 896 and gate/up 4864 x 896) 47.5 / 51.1.
 bool q8k_norm_ok(int tiles16, int nsb, int n_in, int nrows, int nm) {
-  return tiles16 <= 512 && n_in <= 8192 &&
-         std::max(Lds<FMT_Q4K>::bytes(nsb, nrows, nm, n_in), Lds<FMT_Q6K>::bytes(nsb, nrows, nm, n_in)) <= kLdsMax;
+  const size_t lds =
+      std::max(Lds<FMT_Q4K>::bytes(nsb, nrows, nm, n_in), Lds<FMT_Q6K>::bytes(nsb, nrows, nm, n_in));
+  if (n_in > 8192 || lds > kLdsMax) return false;
+  const int per_cu = std::min(std::min((int)(kLdsMax / lds), kMaxWaves / waves_of(nm * nsb)), 2);
+  return tiles16 <= 256 * per_cu;
 }
 
 }  // namespace gemv

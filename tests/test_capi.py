@@ -62,3 +62,27 @@ def test_product_package_does_not_import_oracle():
         if p.suffix in (".py", ".hip", ".cpp", ".h"):
             t = p.read_text()
             assert "oracle" not in t.replace("pagoda_amd", ""), p
+
+
+@pytest.mark.parametrize("tiles16,n_in,rows,nm,fused", [
+    (72, 896, 4, 1, True),      # 4 waves, small LDS
+    (304, 896, 4, 2, True),     # two workgroups of 8 waves per CU
+    (304, 896, 5, 2, False),    # more rows than the few-row kernel's
+    (288, 3584, 1, 1, False),   # 14 waves: one per CU, 32 tiles left for a second round
+    (256, 3584, 1, 2, True),    # one round
+    (512, 2048, 1, 2, False),   # 16 waves
+    (300, 2048, 4, 1, True),    # 71 KB of LDS: two per CU
+    (300, 2048, 5, 1, False),   # 89 KB: one
+    (513, 256, 1, 1, False),
+    (64, 8448, 1, 1, False),    # wider than the ordered-sum norm
+])
+def test_norm_goes_into_launches_of_one_round(tiles16, n_in, rows, nm, fused):
+    """The RMSNorm runs inside a quantized-activation launch only where all its
+    workgroups are resident at once (each repeats the norm's ordered sum): the
+    library's own rule, at the limits of waves, LDS, rows and width."""
+    from pagoda_amd import _lib
+
+    rule = _lib.lib()["_ZN3pgd4gemv16q8act_norm_fusedEiiiiii"]  # pgd::gemv::q8act_norm_fused
+    rule.restype = C.c_bool
+    for fmt in (1, 2):
+        assert rule(fmt, tiles16, (n_in + 255) // 256, n_in, rows, nm) is fused, fmt
