@@ -206,8 +206,8 @@ def test_config4_full_depth_greedy_32_and_batch32(dev, capsys):
 
 def test_config4_widths_prefill_300_tokens(dev):
     """A 300-token prompt at config-4 widths (one 3:1 layer group) is
-    prefilled through the A8 GEMM (weights read once per 128 rows) and the
-    GEMM path's prepared-output emits; logits against the oracle within 1e-3,
+    prefilled through the A8 GEMM (its wide matrices; weights read once per 64
+    rows) and the GEMM path's prepared-output emits; logits against the oracle within 1e-3,
     then 4 greedy decode steps."""
     from dataclasses import replace
 

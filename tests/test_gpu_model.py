@@ -404,9 +404,9 @@ def test_shared_trunk_mixed_decode_and_verify(which, request):
 
 
 def test_long_and_short_prefill_in_one_step(m35):
-    """A 150-token and a 7-token sequence prefilled in one ragged step (the
-    long one's GEMVs take whole 128-row GEMM blocks only through the batch),
-    both against the oracle, then decode."""
+    """A 150-token and a 7-token sequence prefilled in one ragged step (the last
+    GEMV launch of the 157 rows holds rows of both), both against the oracle,
+    then decode."""
     model, oracle = m35
     rng = np.random.default_rng(77)
     long_p, short_p = rng.integers(0, model.cfg.vocab, 150), rng.integers(0, model.cfg.vocab, 7)

@@ -182,7 +182,8 @@ def extreme_blocks(rng, fmt, n_out, n_in):
     (40, 320, 4),       # the most rows of the vector-ALU kernel
     (40, 320, 5),       # the fewest on the matrix cores
     (33, 4864, 6),      # 19 blocks over 10 waves, 6 rows
-    (33, 18944, 2),     # 74 blocks: rows one launch at a time
+    (33, 18944, 2),     # 74 blocks: the most rows whose terms fit the LDS together
+    (33, 18944, 3),     # 74 blocks: rows one launch at a time
     (33040, 256, 1),    # more tiles than workgroups
     (16, 256, 16),      # one subtile, one block, one whole activation tile
     (129, 1280, 17),    # one row into the second activation tile

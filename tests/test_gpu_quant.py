@@ -405,16 +405,16 @@ def test_a8_stream_k_swiglu(dev, n_out, n_in):
 @pytest.mark.parametrize("rows", [256, 300, 390, 516])
 @pytest.mark.parametrize("epi", ["store", "res", "swiglu"])
 def test_a8_prefill_gemm(dev, rows, epi):
-    """Batches of >= 256 rows take the A8 GEMM for their whole 128-row blocks
-    (weights read once per 128 rows) and the GEMV kernels for the rest (44
-    rows at 300, a 6-row partial chunk at 390, a compact 4-row chunk at 516):
-    against fp64 on the same dequantized weights, elementwise, for the store,
-    in-place residual and SwiGLU epilogues; n_out 1000 leaves a partial
-    weight tile."""
+    """Batches of >= 256 rows through the A8 GEMM (a partly filled last block of
+    44 rows at 300, a 6-row chunk at 390) and, for the compact 4-row chunk at
+    516, the GEMV kernels: against fp64 on the same dequantized weights, for
+    the store, in-place residual and SwiGLU epilogues; the last weight block is
+    partly filled, ten groups go round the two stages. A row's bits differ from
+    a 64-row launch's (the GEMV kernels, which split K)."""
     from pagoda_amd import Matrix
     from pagoda_amd.matrix import act_bytes, act_prep_dev
 
-    n_out, K = 1000, 640
+    n_out, K = 4100 if epi == "swiglu" else 8200, 640
     m = Matrix.synth(dev, 0, n_out, K, 61, 3, 0.02)
     u = Matrix.synth(dev, 0, n_out, K, 62, 4, 0.02) if epi == "swiglu" else None
     rng = np.random.default_rng(rows)
@@ -438,28 +438,54 @@ def test_a8_prefill_gemm(dev, rows, epi):
         ref = x64 @ m.dequant().astype(np.float64).T
     got = dev.download(yd, (rows, n_out), np.float32)
     assert rel_err(got, ref) < GEMV_TOL, rel_err(got, ref)
-    for p in (xd, act, yd):
+    y64 = dev.upload(res[:64])
+    act_prep_dev(dev, xd, K, 64, K, act)
+    if epi == "swiglu":
+        Matrix.gemv_swiglu_act_dev(m, u, act, 64, y64, n_out)
+    else:
+        m.gemv_act_dev(act, 64, y64, n_out, y64 if epi == "res" else 0, n_out)
+    assert not np.array_equal(dev.download(y64, (64, n_out), np.float32), got[:64])
+    for p in (xd, act, yd, y64):
         dev.free(p)
 
 
+def gemm_subtiles(n_out, rows, epi):
+    """16-row weight subtiles per wave of that GEMM launch, from the library's
+    own count of its workgroups (64 rows of the batch each)."""
+    import ctypes as C
 
-@pytest.mark.parametrize("n_out,rows,epi", [
-    (8200, 256, "store"),    # 3 subtiles per wave; a partial weight block
-    (8200, 293, "res"),      # a last batch block of 37 rows (its second chunk 5 rows)
-    (8200, 515, "store"),    # 3 rows past whole chunks: the GEMV kernels'
-    (8200, 1030, "res"),     # 4 subtiles per wave; 17 batch blocks (groups of 8, 8 and 1)
-    (4100, 261, "swiglu"),   # the pair, a partial weight block and chunk
-    (4100, 1200, "swiglu"),
+    from pagoda_amd import _lib
+
+    e = {"store": 0, "res": 1, "swiglu": 2}[epi]
+    workgroups = _lib.lib()["_ZN3pgd4gemv18a8_gemm_workgroupsEiii"](n_out, rows, e)
+    subs, blocks = (n_out + 15) // 16, (rows + 63) // 64
+    ns = [n for n in (3, 4) if -(-subs // ((2 if epi == "swiglu" else 4) * n)) * blocks == workgroups]
+    assert len(ns) == 1 and workgroups >= 128, (workgroups, ns)
+    return ns[0]
+
+
+@pytest.mark.parametrize("n_out,K,rows,epi,ns", [
+    (8200, 128, 256, "store", 3),    # 3 subtiles per wave; a partial weight block
+    (8200, 128, 293, "res", 3),      # a last batch block of 37 rows (its second chunk 5 rows)
+    (8200, 128, 515, "store", 3),    # 3 rows past whole chunks: the GEMV kernels'
+    (8200, 128, 1030, "res", 3),     # 17 batch blocks (groups of 8, 8 and 1)
+    (8100, 640, 511, "store", 4),    # 4 subtiles, a partial weight block; ten groups
+    (8100, 640, 511, "res", 4),
+    (8100, 1920, 511, "res", 4),
+    (3832, 128, 1030, "res", 4),     # 17 batch blocks
+    (4100, 128, 261, "swiglu", 4),   # the pair, a partial weight block and chunk
+    (4100, 128, 1200, "swiglu", 4),
 ])
-def test_a8_prefill_gemm_tiles(dev, n_out, rows, epi):
-    """The A8 GEMM at the edges of its tiles (launches of enough workgroups to
-    take it; two groups, so both stages and the fold across groups count):
-    against fp64 on the same dequantized weights, and a row's bits the same
-    whichever launch holds it."""
+def test_a8_prefill_gemm_tiles(dev, n_out, K, rows, epi, ns):
+    """The A8 GEMM at the edges of its tiles and of both its forms, 3 and 4
+    subtiles per wave (launches of enough workgroups to take it; two groups, so
+    both stages and the fold across groups count, or many, so stages are
+    written again): against fp64 on the same dequantized weights, and a row's
+    bits the same whichever launch and form holds it."""
     from pagoda_amd import Matrix
     from pagoda_amd.matrix import act_bytes, act_prep_dev
 
-    K = 128
+    assert gemm_subtiles(n_out, rows - rows % 32 if rows % 32 <= 4 else rows, epi) == ns
     m = Matrix.synth(dev, 0, n_out, K, 71, 3, 0.02)
     u = Matrix.synth(dev, 0, n_out, K, 72, 4, 0.02) if epi == "swiglu" else None
     rng = np.random.default_rng(rows)
@@ -488,6 +514,9 @@ def test_a8_prefill_gemm_tiles(dev, n_out, rows, epi):
     assert rel_err(got, ref) < GEMV_TOL, rel_err(got, ref)
     if rows > 512:
         np.testing.assert_array_equal(run(512).view(np.uint32), got[:512].view(np.uint32))
+    elif ns == 4 and epi != "swiglu":
+        assert gemm_subtiles(n_out, 256, epi) == 3
+        np.testing.assert_array_equal(run(256).view(np.uint32), got[:256].view(np.uint32))
     m.free()
 
 
