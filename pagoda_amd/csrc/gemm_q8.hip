@@ -19,7 +19,7 @@
 // (kStageBytes per 16-row tile and block). q8_mm_kernel: a wave owns 16
 // weight rows, a workgroup of NW waves shares MT 16-row activation tiles,
 // double-buffered through LDS, and walks the K blocks in order; weights go
-// from HBM straight into registers one block ahead.
+// from HBM straight into registers, two blocks ahead (one with two tiles).
 //
 // Bound: the vector ALUs, 64 multiplies and adds per 16 x 16 outputs and
 // block for the ordered sums (32 cycles per MFMA of 16) plus the unpacking,
@@ -52,7 +52,7 @@ typedef uint32_t u4v __attribute__((ext_vector_type(4)));
 // order in which a lane's bytes of the Q6_K planes hold a class.
 constexpr int kSumOff = 8192, kDOff = kSumOff + 512, kStageBytes = kDOff + 64;
 constexpr int kTailUnits = (kStageBytes - kSumOff) / 16;
-// activation rows prepared at a time: bounds the scratch (9.4 MB at K 4096)
+// activation rows prepared at a time: bounds the scratch (9.0 MB at K 4096)
 constexpr int kRowChunk = 1024;
 
 __device__ inline h2 as_h2(uint32_t v) { return __builtin_bit_cast(h2, v); }

@@ -231,17 +231,20 @@ __device__ inline void keep(const GemvArgs& a, int rows, uint32_t sink) {
   if (rows < 0 && sink == 0x9e3779b9u) a.y[0] = 0.0f;
 }
 
-// K blocks of a row in units of 128 weights
-__host__ __device__ inline int k_blocks(const GemvArgs& a) { return a.n_in / 128; }
+// Rows of 36 blocks or more prefetch: a wave of 8 then walks five or more. One
+// row of 896 x 4864 Q8_0 17.3 -> 13.6 us and Q5_0 19.3 -> 15.5, 3584 x 3584 13.9
+// -> 11.1 and 15.2 -> 13.0. Short of that it gives nothing (896 x 2048 Q8_0 7.2
+// and 7.2, Q5_0 8.4 -> 9.1), and 8 rows too wide to share a launch pay it in
+// each (4096 x 12288 Q8_0 251 -> 287).
+__device__ inline bool prefetches(const GemvArgs& a) { return a.n_in / 32 >= 36; }
 
 template <int FMT, int RB, int NW, int EPI>
 __global__ __launch_bounds__(64 * NW) void q8_gemv_kernel(GemvArgs a, int rows) {
   extern __shared__ __attribute__((aligned(16))) char dsm[];
-  // long rows (a wave walks several K blocks): the tile's later blocks are in
-  // the cache by the time the wave reaches them (measured: the 4864-wide down
-  // projection 13.2 -> 11.0 us for Q6_K; tiles of one block per wave lost)
+  // long rows: the tile's later blocks are in the cache by the time a wave
+  // reaches them
   uint32_t sink = 0;
-  if (NW == 8 && k_blocks(a) > 8) {
+  if (NW == 8 && prefetches(a)) {
     prefetch_tile<FMT>(a, false, blockIdx.x, 64 * NW, sink);
     if constexpr (EPI == EPI_SWIGLU) prefetch_tile<FMT>(a, true, blockIdx.x, 64 * NW, sink);
   }
@@ -262,7 +265,7 @@ __global__ __launch_bounds__(64 * NW) void q8_pair_kernel(GemvArgs a, GemvArgs b
   extern __shared__ __attribute__((aligned(16))) char dsm[];
   const bool first = (int)blockIdx.x < split;
   uint32_t sink = 0;
-  if (NW == 8 && k_blocks(a) > 8) {
+  if (NW == 8 && prefetches(a)) {
     if (first) prefetch_tile<FMT>(a, false, blockIdx.x, 64 * NW, sink);
     else prefetch_tile<FMT2>(b, false, blockIdx.x - split, 64 * NW, sink);
   }
@@ -301,10 +304,13 @@ void launch_q8(GemvArgs a, int nrows, hipStream_t s) {
 }
 
 // waves per workgroup from the K blocks of a row (the sums do not depend on
-// it: every block's terms are added in block order by one lane)
+// it: every block's terms are added in block order by one lane): four walk at
+// most five blocks each, from 20 blocks on eight
+constexpr int kEightWaveBlocks = 20;
+
 template <int FMT, int RB, int EPI>
 void launch_waves(const GemvArgs& a, int nrows, hipStream_t s) {
-  if (k_blocks(a) <= 4) return launch_q8<FMT, RB, 4, EPI>(a, nrows, s);
+  if (a.n_in / 32 < kEightWaveBlocks) return launch_q8<FMT, RB, 4, EPI>(a, nrows, s);
   launch_q8<FMT, RB, 8, EPI>(a, nrows, s);
 }
 
@@ -384,10 +390,9 @@ void launch_pair_q8(GemvArgs a, GemvArgs b, int nrows, hipStream_t s) {
 // matrices: they have the same K)
 template <int FMT, int FMT2>
 void pair_rows(const GemvArgs& a, const GemvArgs& b, int nrows, hipStream_t s) {
-  const int kb = k_blocks(a);
   auto go = [&](auto rb) {
     constexpr int RB = decltype(rb)::value;
-    if (kb <= 4) return launch_pair_q8<FMT, FMT2, RB, 4>(a, b, nrows, s);
+    if (a.n_in / 32 < kEightWaveBlocks) return launch_pair_q8<FMT, FMT2, RB, 4>(a, b, nrows, s);
     launch_pair_q8<FMT, FMT2, RB, 8>(a, b, nrows, s);
   };
   const size_t cap = 160 * 1024;
