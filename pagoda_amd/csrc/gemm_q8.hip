@@ -523,6 +523,14 @@ std::mutex g_operands;
 
 }  // namespace
 
+// Microseconds of up to 16 rows: both launches and the K chain, once per round
+// of a workgroup on each CU (a second one of any size counts 0.6). Measured
+// over the same shapes as q8k_us, within 10% up to 1024 tiles.
+double q8_gemm_us(int fmt, int tiles16, int nsb) {
+  const double rounds = tiles16 / 4 / 256.0;
+  return 5.9 + (fmt == FMT_Q4K ? 0.76 : 1.1) * nsb * (rounds <= 1.0 ? 1.0 : std::max(1.6, 0.92 * rounds));
+}
+
 void run_q8_gemm(int fmt, GemvArgs a, int nrows, int epi, hipStream_t s) {
   for (int r0 = 0; r0 < nrows; r0 += kRowChunk) {
     const int rows = min(kRowChunk, nrows - r0);

@@ -464,6 +464,12 @@ void run_q8k_gemv(int fmt, const GemvArgs& a, int nrows, int epi, hipStream_t s)
 void run_q8k_gemv_pair(int fmt_a, const GemvArgs& a, int fmt_b, const GemvArgs& b, int nrows, hipStream_t s);
 void run_q8_gemm(int fmt, GemvArgs a, int nrows, int epi, hipStream_t s);
 void run_q8_gemm_pair(int fmt_a, GemvArgs a, int fmt_b, GemvArgs b, int nrows, hipStream_t s);
+// their estimated microseconds (nm matrices of tiles16 16-row tiles; the GEMM's
+// tiles of all of them, at most 16 rows), and whether the first takes a launch
+// of nrows rows: where it is no slower by more than slack us
+double q8k_us(int fmt, int tiles16, int nsb, int nrows, int nm);
+double q8_gemm_us(int fmt, int tiles16, int nsb);
+bool q8act_few_rows(int fmt, int tiles16, int nsb, int nrows, int nm, double slack = 0.0);
 // two store GEMVs of one input in one launch (formats of one activation type)
 bool q8act_pair_ok(int fmt_a, int fmt_b);
 void run_q8act_pair(int fmt_a, const GemvArgs& a, int fmt_b, const GemvArgs& b, int nrows, hipStream_t s);

@@ -328,17 +328,8 @@ void launch_rows(const GemvArgs& a, int nrows, hipStream_t s) {
   launch_waves<FMT, 1, EPI>(a, nrows, s);
 }
 
-// The most rows a Q4_K / Q6_K launch runs in gemv_q8k.hip; more go to the
-// matrix cores (gemm_q8.hip). A row costs the former about 0.4 us plus 0.11 us
-// per K block, the latter takes about 5 us plus 1 us per K block whatever the
-// rows. Measured us (former / latter): 4864 x 896 4 rows 7.8 / 8.7, 5 rows
-// 9.1 / 8.9; 2159 x 2496 6 rows 11.5 / 13.3; 896 x 4864 Q6_K 6 rows 21 / 26.
-// Matrices with enough tiles to fill the chip pay the former's instructions
-// per row instead: 18944 x 3584 2 rows 31 / 22, 30000 x 1024 11.9 / 10.9.
-int gemv_rows(int tiles16, int nsb) {
-  if ((long long)tiles16 * nsb > 4096) return 1;
-  return nsb >= 8 ? 6 : 4;
-}
+// The most rows a Q4_K / Q6_K launch runs in gemv_q8k.hip.
+constexpr int kFewRows = 6;
 
 // The widest rows Q4_K / Q6_K launches take, the same for every row count: one
 // quantized row and the block terms of 32 outputs in 160 KiB.
@@ -354,9 +345,9 @@ void dispatch(int fmt, const GemvArgs& a, int nrows, hipStream_t s) {
     case FMT_Q6K:
       PGD_CHECK(k256_fits(fmt, a.nsb, EPI == EPI_SWIGLU ? 2 : 1), kErrShape,
                 "activation rows too wide for the quantized-activation GEMV");
-      if (nrows > gemv_rows((EPI == EPI_SWIGLU ? 2 : 1) * ((a.n_out + 15) / 16), a.nsb))
-        return run_q8_gemm(fmt, a, nrows, EPI, s);
-      return run_q8k_gemv(fmt, a, nrows, EPI, s);
+      if (a.nw || q8act_few_rows(fmt, (a.n_out + 15) / 16, a.nsb, nrows, EPI == EPI_SWIGLU ? 2 : 1))
+        return run_q8k_gemv(fmt, a, nrows, EPI, s);
+      return run_q8_gemm(fmt, a, nrows, EPI, s);
     case FMT_Q8_0: return launch_rows<FMT_Q8_0, EPI>(a, nrows, s);
     case FMT_Q5_0: return launch_rows<FMT_Q5_0, EPI>(a, nrows, s);
   }
@@ -410,12 +401,24 @@ bool q8act_pair_ok(int fmt_a, int fmt_b) {
   return (k256(fmt_a) && k256(fmt_b)) || (b32(fmt_a) && b32(fmt_b));
 }
 
+// Same bits either way; the estimates of both say which is faster. us, few-row
+// kernel / matrix cores: 5120 x 5120 Q4_K 2 rows 13.8 / 20.9, 4 rows 26.1 / 20.9
+// (two workgroups no longer fit a CU's LDS); 3840 x 5120 6 rows 18.9 / 21.0;
+// 2048 x 11008 2 rows 14.4 / 38.1, 5 rows 48.4 / 38.2 (rows one at a time);
+// 18944 x 3584 2 rows 29.8 / 21.1; 4864 x 896 4 rows 7.6 / 8.8.
+bool q8act_few_rows(int fmt, int tiles16, int nsb, int nrows, int nm, double slack) {
+  if (nrows <= 1) return true;
+  return nrows <= kFewRows && q8k_us(fmt, tiles16, nsb, nrows, nm) <= q8_gemm_us(fmt, nm * tiles16, nsb) + slack;
+}
+
 // An RMSNorm launch of one 896-wide row takes 6.0 us, of which the GEMV launch
 // repeats about 4.5 (q|k + v 5.2 -> 9.5 us, gate/up 7.5 -> 12.8 us with the
-// norm inside); a decode step of the 0.5B model 1271 -> 1139 us.
+// norm inside); a decode step of the 0.5B model 1271 -> 1139 us. So the fused
+// launch may be slower than the matrix cores by 2.7: gate/up 4864 x 896 4 rows
+// 15.0 us against 16.1 with a norm launch, 5 rows 17.6 against 16.1.
 bool q8act_norm_fused(int fmt, int tiles16, int nsb, int n_in, int nrows, int nm) {
-  return (fmt == FMT_Q4K || fmt == FMT_Q6K) && nrows <= gemv_rows(nm * tiles16, nsb) &&
-         k256_fits(fmt, nsb, nm) && q8k_norm_ok(tiles16, nsb, n_in, nrows, nm);
+  return (fmt == FMT_Q4K || fmt == FMT_Q6K) && k256_fits(fmt, nsb, nm) &&
+         q8act_few_rows(fmt, tiles16, nsb, nrows, nm, 2.7) && q8k_norm_ok(tiles16, nsb, n_in, nrows, nm);
 }
 
 void run_q8act_pair(int fmt_a, const GemvArgs& a, int fmt_b, const GemvArgs& b, int nrows, hipStream_t s) {
@@ -424,9 +427,9 @@ void run_q8act_pair(int fmt_a, const GemvArgs& a, int fmt_b, const GemvArgs& b, 
   if (fmt_a == FMT_Q4K || fmt_a == FMT_Q6K) {
     PGD_CHECK(k256_fits(fmt_a, a.nsb, 1) && k256_fits(fmt_b, b.nsb, 1), kErrShape,
               "activation rows too wide for the quantized-activation GEMV");
-    if (nrows > gemv_rows((a.n_out + 15) / 16 + (b.n_out + 15) / 16, a.nsb))
-      return run_q8_gemm_pair(fmt_a, a, fmt_b, b, nrows, s);
-    return run_q8k_gemv_pair(fmt_a, a, fmt_b, b, nrows, s);
+    if (a.nw || q8act_few_rows(fmt_a, (a.n_out + 15) / 16 + (b.n_out + 15) / 16, a.nsb, nrows, 1))
+      return run_q8k_gemv_pair(fmt_a, a, fmt_b, b, nrows, s);
+    return run_q8_gemm_pair(fmt_a, a, fmt_b, b, nrows, s);
   }
 #define PGD_PAIR(F1, F2) \
   if (fmt_a == F1 && fmt_b == F2) return pair_rows<F1, F2>(a, b, nrows, s);

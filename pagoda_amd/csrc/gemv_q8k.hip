@@ -522,6 +522,25 @@ void run_q8k_gemv_pair(int fmt_a, const GemvArgs& a, int fmt_b, const GemvArgs& 
   else run_pair<FMT_Q6K, FMT_Q6K>(a, b, nrows, s);
 }
 
+// Microseconds of run_q8k_gemv. The workgroups of a CU share its issue slots (24
+// waves of these kernels fit, by 80 registers; one of 14 waves or more, or one
+// that fills the LDS, has the CU to itself), a row costs about as much per K
+// block in each; rows that do not fit the LDS together run one launch each.
+// Fitted to 33 shapes of 256..152064 x 896..18944 in both formats at 1..8 rows:
+// 3% off in the median. What q8act_few_rows chooses by it is 0.1% slower than
+// the faster of both on average, 8% at most but for 152064 x 896 (21%, 2 rows).
+double q8k_us(int fmt, int tiles16, int nsb, int nrows, int nm) {
+  auto need = [&](int rb) {
+    return fmt == FMT_Q4K ? Lds<FMT_Q4K>::bytes(nsb, rb, nm) : Lds<FMT_Q6K>::bytes(nsb, rb, nm);
+  };
+  if (nrows > 1 && need(nrows) > kLdsMax) return nrows * q8k_us(fmt, tiles16, nsb, 1, nm);
+  const int nw = waves_of(nm * nsb);
+  const int per_cu = std::max(1, std::min((int)(kLdsMax / need(nrows)), 24 / nw));
+  const double blocks = (fmt == FMT_Q4K ? 1.0 : 1.3) * nm * nsb;
+  const double one = 2.4 + 0.07 * blocks + nrows * ((nm * nsb <= kMaxWaves ? 0.55 : 1.15) + 0.065 * blocks);
+  return 1.0 + one * (1.0 + std::max(0.93 / per_cu, nw / 17.5) * ((tiles16 + 255) / 256 - 1));
+}
+
 // Every workgroup of a launch with the norm repeats the chain of n_in additions,
 // so the norm goes in only where all of them are resident at once: per CU the
 // LDS, and 16 waves (the kernels' 128 registers), at most two. A second round

@@ -86,3 +86,26 @@ def test_norm_goes_into_launches_of_one_round(tiles16, n_in, rows, nm, fused):
     rule.restype = C.c_bool
     for fmt in (1, 2):
         assert rule(fmt, tiles16, (n_in + 255) // 256, n_in, rows, nm) is fused, fmt
+
+
+@pytest.mark.parametrize("fmt,n_out,n_in,few", [
+    (1, 5120, 5120, 3),     # two workgroups per CU; the rows of 4 fill the LDS
+    (2, 5120, 5120, 3),
+    (1, 3840, 5120, 6),     # one workgroup per CU
+    (1, 18944, 3584, 1),    # five workgroups of 14 waves per CU
+    (1, 2048, 11008, 3),    # 4 rows do not fit the LDS: one launch each
+    (2, 2048, 11008, 4),
+    (1, 3584, 18944, 4),
+    (1, 4864, 896, 4),
+    (1, 152064, 896, 1),
+])
+def test_few_row_kernel_takes_the_rows_it_is_faster_for(fmt, n_out, n_in, few):
+    """The most rows of a Q4_K / Q6_K launch that run in the few-row kernel
+    instead of on the matrix cores (same bits): the library's own rule, where
+    the measured times of both cross."""
+    from pagoda_amd import _lib
+
+    rule = _lib.lib()["_ZN3pgd4gemv14q8act_few_rowsEiiiiid"]  # pgd::gemv::q8act_few_rows
+    rule.restype, rule.argtypes = C.c_bool, [C.c_int] * 5 + [C.c_double]
+    got = [rule(fmt, (n_out + 15) // 16, (n_in + 255) // 256, r, 1, 0.0) for r in range(1, 9)]
+    assert got == [r <= few for r in range(1, 9)], got

@@ -179,8 +179,13 @@ def extreme_blocks(rng, fmt, n_out, n_in):
 @pytest.mark.parametrize("fmt", [1, 2])
 @pytest.mark.parametrize("n_out,n_in,rows", [
     (40, 320, 1),       # one row; a K tail; partly filled weight tile
-    (40, 320, 4),       # the most rows of the vector-ALU kernel
-    (40, 320, 5),       # the fewest on the matrix cores
+    (40, 320, 4),
+    (40, 320, 5),       # five and six rows of the vector-ALU kernel
+    (40, 320, 6),
+    (40, 320, 7),       # the fewest on the matrix cores
+    (4000, 5120, 2),    # 20 blocks over 10 waves, two per wave
+    (1000, 5120, 6),
+    (9728, 512, 2),     # 608 tiles: the matrix cores from 4 rows on
     (33, 4864, 6),      # 19 blocks over 10 waves, 6 rows
     (33, 18944, 2),     # 74 blocks: the most rows whose terms fit the LDS together
     (33, 18944, 3),     # 74 blocks: rows one launch at a time
